@@ -1355,14 +1355,6 @@ void StateVector::collapse(uint32_t wire, bool branch) {
     normalize();
 }
 
-std::vector<double> StateVector::reduce_rows_to_host(uint32_t rows, uint32_t cols) {
-    slots_.ensure(static_cast<size_t>(cols) * sizeof(double));
-    launch_reduce_rows(static_cast<const double *>(partials_.p), rows, cols, static_cast<double *>(slots_.p), stream_);
-    std::vector<double> h(cols);
-    read_back(h.data(), slots_.p, cols * sizeof(double));
-    return h;
-}
-
 std::vector<double> StateVector::probs(const uint32_t *wires, int nw, bool all) {
     if (!all && nw == 0) return {1.0};
     std::vector<int> bits;
@@ -1374,21 +1366,18 @@ std::vector<double> StateVector::probs(const uint32_t *wires, int nw, bool all) 
     }
     const int m = static_cast<int>(bits.size());
     flush();
-    if (m > 12) {
-        slots_.ensure(sizeof(double) << m);
-        dispatch(dtype_, [&](auto t) {
-            launch_probs_gather<decltype(t)>(data(), n_, bits.data(), m, static_cast<double *>(slots_.p), stream_);
-        });
-        std::vector<double> h(static_cast<size_t>(1) << m);
-        read_back(h.data(), slots_.p, h.size() * sizeof(double));
-        return h;
+    const uint32_t rows = probs_rows(n_, bits.data(), m);
+    slots_.ensure(sizeof(double) << m);
+    double *out = static_cast<double *>(slots_.p), *part = out;
+    if (rows > 1) {
+        partials_.ensure((static_cast<size_t>(rows) * sizeof(double)) << m);
+        part = static_cast<double *>(partials_.p);
     }
-    const uint32_t nb = static_cast<uint32_t>(std::min<uint64_t>(512, std::max<uint64_t>(1, length() / 1024)));
-    partials_.ensure((static_cast<size_t>(nb) * sizeof(double)) << m);
-    dispatch(dtype_, [&](auto t) {
-        launch_probs_hist<decltype(t)>(data(), n_, bits.data(), m, static_cast<double *>(partials_.p), nb, stream_);
-    });
-    return reduce_rows_to_host(nb, 1u << m);
+    dispatch(dtype_, [&](auto t) { launch_probs<decltype(t)>(data(), n_, bits.data(), m, part, stream_); });
+    if (rows > 1) launch_reduce_rows(part, rows, 1u << m, out, stream_);
+    std::vector<double> h(static_cast<size_t>(1) << m);
+    read_back(h.data(), out, h.size() * sizeof(double));
+    return h;
 }
 
 double StateVector::expval_named(const std::string &name, const uint32_t *wires, int nw) {

@@ -351,7 +351,6 @@ class StateVector {
     hipEvent_t take_event();
 
     int kt_for(int ns) const;
-    std::vector<double> reduce_rows_to_host(uint32_t rows, uint32_t cols);
     void apply_obs_inplace(const Obs &o, void *state, std::vector<LOp> &prog);
     // Re<psi|O psi> and <O psi|O psi> of a dense k-wire operator, one read pass
     void dense_moments(std::vector<cd> m, const uint32_t *wires, int nw, double *mean, double *mean_square);

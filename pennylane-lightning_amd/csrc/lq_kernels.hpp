@@ -81,14 +81,12 @@ void launch_overlap(const void *a, int dtype_a, const void *b, int dtype_b, int 
 template <typename T>
 void launch_sparse_rows(const void *a, void *out, const int64_t *indptr, const int64_t *indices, const void *values,
                         uint64_t nrows, int mode, double2 *partials, uint32_t nblocks, hipStream_t s);
-// marginal probabilities: out[o] over the wires given as physical bits
-// (bits[0] is the output MSB). Small nw: per-block LDS histograms into
-// partials[block][o]; large nw: one output per thread.
-template <typename T>
-void launch_probs_hist(const void *a, int n, const int *bits, int nw, double *partials,
-                       uint32_t nblocks, hipStream_t s);
-template <typename T>
-void launch_probs_gather(const void *a, int n, const int *bits, int nw, double *out, hipStream_t s);
+// marginal probabilities over the wires given as physical bits (bits[0] is
+// the output MSB): out[row][o], o < 2^nw, for probs_rows() rows whose sum is
+// the result (one row: out is the result); at most 2^19 entries when there is
+// more than one row
+uint32_t probs_rows(int n, const int *bits, int nw);
+template <typename T> void launch_probs(const void *a, int n, const int *bits, int nw, double *out, hipStream_t s);
 void launch_reduce_rows(const double *partials, uint32_t nrows, uint32_t ncols, double *out,
                         hipStream_t s);
 

@@ -1,16 +1,16 @@
 // Probabilities of a state held in caller-owned device memory, with the
-// per-block partial histograms in a fixed device array instead of memory
-// the library allocates: for callers that cannot allocate (code under HIP
-// graph capture, tight serving loops). The kernels are the ones lq_probs
-// runs (LDS histogram per block, then a compensated sum of the rows).
+// rows of partial sums in a fixed device array instead of memory the library
+// allocates: for callers that cannot allocate (code under HIP graph capture,
+// tight serving loops). The kernels are the ones lq_probs runs (sums over the
+// unmeasured bits, split over rows when there are few outputs, then a
+// compensated sum of the rows).
 //
 // The array `scratch` is a file-scope __device__ variable: each GPU holds its
 // own copy until the process ends. Its name in host code is not a device
 // address; the address is taken once per device with hipGetSymbolAddress
 // (with that device current) and only that pointer is passed to kernels.
-// Every probs block writes its whole row of partials, so nothing needs
-// clearing between calls; calls that overlap on one GPU share the array and
-// race.
+// The probs kernel writes every entry of its rows, so nothing needs clearing
+// between calls; calls that overlap on one GPU share the array and race.
 #include <hip/hip_runtime.h>
 
 #include <mutex>
@@ -21,8 +21,8 @@
 namespace lqamd {
 namespace {
 
-constexpr uint32_t kRows = 512; // histogram blocks, as lq_probs uses at most
-static __device__ __align__(256) double scratch[static_cast<size_t>(kRows) << kNoAllocProbsMaxWires];
+constexpr size_t kEntries = 1u << 19; // rows times outputs, as launch_probs writes at most
+static __device__ __align__(256) double scratch[kEntries];
 
 constexpr int kMaxDevices = 64;
 std::mutex g_mu;
@@ -61,13 +61,12 @@ void probs_noalloc(const void *state, int n, int dtype, const uint32_t *wires, i
         seen |= 1ull << b;
         bits[j] = b;
     }
-    double *part = scratch_on_current_device();
-    // the block count lq_probs uses for this size (one row of partials each)
-    const uint64_t len = 1ull << n;
-    const uint32_t nb = static_cast<uint32_t>(len / 1024 < 1 ? 1 : (len / 1024 > kRows ? kRows : len / 1024));
-    if (dtype) launch_probs_hist<double>(state, n, bits, nw, part, nb, s);
-    else launch_probs_hist<float>(state, n, bits, nw, part, nb, s);
-    launch_reduce_rows(part, nb, 1u << nw, out, s);
+    const uint32_t rows = probs_rows(n, bits, nw);
+    LQ_ABORT_IF(rows > 1 && (static_cast<size_t>(rows) << nw) > kEntries, "too many rows of partial probabilities");
+    double *part = rows > 1 ? scratch_on_current_device() : out;
+    if (dtype) launch_probs<double>(state, n, bits, nw, part, s);
+    else launch_probs<float>(state, n, bits, nw, part, s);
+    if (rows > 1) launch_reduce_rows(part, rows, 1u << nw, out, s);
     hip_check(hipGetLastError(), "probs launch");
 }
 
