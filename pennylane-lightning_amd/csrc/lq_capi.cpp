@@ -204,7 +204,8 @@ int lq_sv_dlpack(lq_sv_t sv, void **out) {
     return guard([&] {
         LQ_ABORT_IF(out == nullptr, "null argument");
         StateVector &s = S(sv);
-        void *p = s.data(); // executes a deferred reset's write first
+        s.flush();          // first: the queued gates' first pass forms a deferred reset itself
+        void *p = s.data(); // writes one that is left
         s.synchronize();
         hipPointerAttribute_t attr{};
         hip_check(hipPointerGetAttributes(&attr, p), "hipPointerGetAttributes");
