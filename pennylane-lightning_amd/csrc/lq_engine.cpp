@@ -147,6 +147,22 @@ LOp identity_dot(uint32_t sa, uint32_t sb, int slot) {
 // Pauli word as the cheapest op form for a dot: a parity op for Z-only
 // words, a dense 2x2 / 4x4 (or diagonal) op for words on one or two qubits,
 // the general Pauli-string op otherwise.
+// Kernel terms of a Pauli sum, in order of x (launch_pauli_sum). For an
+// expectation only the real part of a word's coefficient counts, and words
+// with x != 0 count twice for half of the index pairs.
+std::vector<PauliTerm> pauli_terms(const std::vector<PauliWord> &words, bool expectation) {
+    std::vector<PauliTerm> terms;
+    terms.reserve(words.size());
+    for (const auto &w : words) {
+        cd c = expectation ? cd(w.coeff.real() * (w.x ? 2.0 : 1.0), 0.0) : w.coeff;
+        // times (-i)^ny, component by component so that zeros stay exact
+        for (int i = 0; i < (w.ny & 3); ++i) c = cd(c.imag(), -c.real());
+        terms.push_back({w.x, w.yz, c.real(), c.imag()});
+    }
+    std::stable_sort(terms.begin(), terms.end(), [](const PauliTerm &a, const PauliTerm &b) { return a.x < b.x; });
+    return terms;
+}
+
 LOp pauli_dot_op(int n, const PauliWord &w) {
     (void)n;
     const uint64_t sup = w.x | w.yz;
@@ -1496,17 +1512,12 @@ void StateVector::apply_obs_to(const Obs &o, const void *in, void *out) {
     }
     std::vector<PauliWord> words;
     if (obs_to_pauli(o, n_, &words)) {
-        std::vector<PauliTerm> terms;
-        for (const auto &w : words) {
-            cd c = w.coeff;
-            for (int i = 0; i < (w.ny & 3); ++i) c *= cd(0, -1);
-            terms.push_back({w.x, w.yz, c.real(), c.imag()});
-        }
+        const std::vector<PauliTerm> terms = pauli_terms(words, false);
         small_.ensure(terms.size() * sizeof(PauliTerm) + 256);
         upload_small(small_.p, small_.bytes, terms.data(), terms.size() * sizeof(PauliTerm));
         dispatch(dtype_, [&](auto t) {
             launch_pauli_sum<decltype(t)>(in, out, static_cast<const PauliTerm *>(small_.p),
-                                          static_cast<uint32_t>(terms.size()), n_, 1, nullptr, 0, stream_);
+                                          static_cast<uint32_t>(terms.size()), n_, 1, nullptr, stream_);
         });
         hip_check(hipStreamSynchronize(stream_), "sync");
         return;
@@ -1577,20 +1588,15 @@ double StateVector::expval_obs(const Obs &o) {
             for (size_t i = 0; i < words.size(); ++i) e += (words[i].coeff * v[i]).real();
             return e;
         }
-        std::vector<PauliTerm> terms;
-        for (const auto &w : words) {
-            cd c = w.coeff;
-            for (int i = 0; i < (w.ny & 3); ++i) c *= cd(0, -1);
-            terms.push_back({w.x, w.yz, c.real(), c.imag()});
-        }
+        const std::vector<PauliTerm> terms = pauli_terms(words, true);
         small_.ensure(terms.size() * sizeof(PauliTerm) + 256);
         upload_small(small_.p, small_.bytes, terms.data(), terms.size() * sizeof(PauliTerm));
-        const uint32_t nb = static_cast<uint32_t>(std::min<uint64_t>(1024, std::max<uint64_t>(1, length() / 256)));
+        const uint32_t nb = pauli_blocks(n_, 0);
         partials_.ensure(nb * sizeof(double2));
         dispatch(dtype_, [&](auto t) {
             launch_pauli_sum<decltype(t)>(data(), nullptr, static_cast<const PauliTerm *>(small_.p),
                                           static_cast<uint32_t>(terms.size()), n_, 0,
-                                          static_cast<double2 *>(partials_.p), nb, stream_);
+                                          static_cast<double2 *>(partials_.p), stream_);
         });
         std::vector<double2> h(nb);
         read_back(h.data(), partials_.p, nb * sizeof(double2));

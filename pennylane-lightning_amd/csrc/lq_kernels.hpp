@@ -62,11 +62,14 @@ template <typename T> void launch_tile_reg(const TileRegArgs &a, size_t lds_byte
 void launch_reduce_slots(const double2 *partials, const SlotRange *ranges, uint32_t nslots,
                          double2 *out, hipStream_t s);
 
-// mode 0: partials[block] = sum_t c_t sum_i conj(a[i]) P_t a[i]   (expectation)
-// mode 1: out[i] = sum_t c_t (P_t a)[i]                             (apply)
+// Terms sorted by x. mode 0: partials[block].x, block < pauli_blocks(n, 0), adds
+// up to Re sum_t c_t sum_i conj(a[i]) P_t a[i] (expectation; terms Hermitian,
+// coefficients of terms with x != 0 doubled, see pauli_sum_kernel)
+// mode 1: out[i] = sum_t c_t (P_t a)[i] (apply)
+uint32_t pauli_blocks(int n, int mode);
 template <typename T>
 void launch_pauli_sum(const void *a, void *out, const PauliTerm *terms, uint32_t nterms, int n,
-                      int mode, double2 *partials, uint32_t nblocks, hipStream_t s);
+                      int mode, double2 *partials, hipStream_t s);
 
 // sum_i |a_i|^2 into per-block partials
 template <typename T>
