@@ -721,6 +721,7 @@ StateVector::Planned StateVector::plan(const std::vector<LOp> &prog, int ns, boo
     cfg.kt_max = kt_for(ns);
     cfg.low_bits = t.low_bits >= 0 ? t.low_bits : (dtype_ ? 4 : 5);
     cfg.budget = t.budget > 0 ? t.budget : 24.0;
+    cfg.dense_passes = true;
     // register-resident passes for tiles of 11 or 12 bits with one or two states
     const int ktr = std::min(cfg.kt_max, 8 + kMaxRegBits);
     if (t.reg && ns <= 2 && n_ >= 11 && ktr >= 11) {
@@ -833,6 +834,26 @@ StateVector::Planned StateVector::plan(const std::vector<LOp> &prog, int ns, boo
     return out;
 }
 
+StateVector::Pending StateVector::profile_begin(const PassPlan &pp, double states, bool specialised) {
+    Pending pe{};
+    pe.a = take_event();
+    pe.b = take_event();
+    pe.bytes = static_cast<double>(bytes()) * states;
+    pe.rec.ops = static_cast<uint32_t>(pp.ops.size());
+    pe.rec.stages = static_cast<uint32_t>(pp.stages.size());
+    pe.rec.transposes = pp.end_transpose ? 1u : 0u;
+    for (const TileStage &st : pp.stages) pe.rec.transposes += st.entry == ENTRY_TRANSPOSE;
+    pe.rec.specialised = specialised ? 1u : 0u;
+    for (int b : pp.tbits) pe.rec.tile_bits |= 1ull << b;
+    hip_check(hipEventRecord(pe.a, stream_), "hipEventRecord");
+    return pe;
+}
+
+void StateVector::profile_end(const Pending &pe) {
+    hip_check(hipEventRecord(pe.b, stream_), "hipEventRecord");
+    pending_.push_back(pe);
+}
+
 std::vector<cd> StateVector::execute(const Planned &pl, const std::vector<void *> &states, int nslots) {
     std::vector<cd> result(static_cast<size_t>(nslots), 0.0);
     const int ns = static_cast<int>(states.size());
@@ -937,6 +958,21 @@ std::vector<cd> StateVector::execute(const Planned &pl, const std::vector<void *
     char *dp = static_cast<char *>(pbuf.p);
     for (size_t p = 0; p < passes.size(); ++p) {
         const PassPlan &pp = passes[p];
+        if (pp.dense) {
+            DenseTileArgs da = dense_tile_args(pp, n_);
+            int cnt = 0;
+            for (int s = 0; s < ns; ++s)
+                if ((pp.store_mask >> s) & 1u) da.sv[cnt++] = states[s];
+            const double2 *u = reinterpret_cast<const double2 *>(dp + coef_at) + coef_off[p];
+            Pending pe{};
+            if (prof) pe = profile_begin(pp, 2.0 * cnt, false);
+            dispatch(dtype_, [&](auto tt) {
+                launch_dense_tile<decltype(tt)>(da, static_cast<int>(pp.ops[0].k), cnt, u, stream_);
+            });
+            ++generic_passes_;
+            if (prof) profile_end(pe);
+            continue;
+        }
         TilePassArgs a{};
         for (int s = 0; s < ns; ++s) a.sv[s] = states[s];
         a.ops = reinterpret_cast<const TileOp *>(dp + op_off[p]);
@@ -974,18 +1010,9 @@ std::vector<cd> StateVector::execute(const Planned &pl, const std::vector<void *
         }
         Pending pe{};
         if (prof) {
-            pe.a = take_event();
-            pe.b = take_event();
             // a pass that forms a deferred reset reads nothing of that state
             const int reads = __builtin_popcount(pp.load_mask) - ((p == 0 && form_basis) ? 1 : 0);
-            pe.bytes = static_cast<double>(bytes()) * (reads + __builtin_popcount(pp.store_mask));
-            pe.rec.ops = static_cast<uint32_t>(pp.ops.size());
-            pe.rec.stages = static_cast<uint32_t>(pp.stages.size());
-            pe.rec.transposes = pp.end_transpose ? 1u : 0u;
-            for (const TileStage &st : pp.stages) pe.rec.transposes += st.entry == ENTRY_TRANSPOSE;
-            pe.rec.specialised = fns[p] ? 1u : 0u;
-            for (int b : pp.tbits) pe.rec.tile_bits |= 1ull << b;
-            hip_check(hipEventRecord(pe.a, stream_), "hipEventRecord");
+            pe = profile_begin(pp, reads + __builtin_popcount(pp.store_mask), fns[p] != nullptr);
         }
         if (fns[p])
             jit_launch(fns[p], dtype_, ra.sv[0], ra.sv[1], ra.sv[2], ra.sv[3], ra.coef, ra.partials, ra.ntiles,
@@ -993,10 +1020,7 @@ std::vector<cd> StateVector::execute(const Planned &pl, const std::vector<void *
         else if (pp.reg) dispatch(dtype_, [&](auto tt) { launch_tile_reg<decltype(tt)>(ra, lds, stream_); });
         else dispatch(dtype_, [&](auto tt) { launch_tile_pass<decltype(tt)>(a, lds, stream_); });
         ++(fns[p] ? jit_passes_ : generic_passes_);
-        if (prof) {
-            hip_check(hipEventRecord(pe.b, stream_), "hipEventRecord");
-            pending_.push_back(pe);
-        }
+        if (prof) profile_end(pe);
     }
     hip_check(hipGetLastError(), "tile pass launch");
     if (nslots > 0) {

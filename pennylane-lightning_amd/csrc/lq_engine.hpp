@@ -343,6 +343,9 @@ class StateVector {
         double bytes;
         PassRecord rec;
     };
+    // events around a launch of `pp` that moves `states` states; end() logs it
+    Pending profile_begin(const PassPlan &pp, double states, bool specialised);
+    void profile_end(const Pending &pe);
     std::vector<PassRecord> pass_log_;
     std::vector<Pending> pending_;
     std::vector<hipEvent_t> ev_free_;

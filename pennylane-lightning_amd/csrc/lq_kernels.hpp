@@ -58,6 +58,25 @@ struct TileRegArgs {
 };
 template <typename T> void launch_tile_reg(const TileRegArgs &a, size_t lds_bytes, hipStream_t s);
 
+// In place, on `ns` states: a dense operator on k = 3..6 bits (lq_dense.hip).
+// A tile of kDenseTileBits bits (tb, ascending; the targets among them) is
+// held as a 2^k x 2^(kDenseTileBits - k) panel; lp[b] is the bit of the panel
+// coordinate row * columns + column that tile bit b stands for. Control bits
+// outside the tile are fixed in ocval and are not among the outside bits ob.
+constexpr int kDenseTileBits = 11;
+struct DenseTileArgs {
+    void *sv[kMaxStates];
+    uint64_t ntiles;          // 2^nout
+    uint64_t ocval;
+    uint32_t ccmask, ccval;   // controls inside the tile, on column bits
+    int32_t nout;
+    int32_t tb[kDenseTileBits];
+    int32_t lp[kDenseTileBits];
+    int32_t ob[kMaxOutsideBits];
+};
+// U: row-major 2^k x 2^k complex double on the device
+template <typename T> void launch_dense_tile(const DenseTileArgs &a, int k, int ns, const double2 *U, hipStream_t s);
+
 // out[slot] = sum of partials (Neumaier-compensated, fixed order)
 void launch_reduce_slots(const double2 *partials, const SlotRange *ranges, uint32_t nslots,
                          double2 *out, hipStream_t s);

@@ -10,6 +10,7 @@
 // are read-only dots. A pass greedily takes ready ops whose non-diagonal bits
 // fit in its tile (at most kt_max bits, the low bits always included), up to
 // a compute budget; diagonal ops fit any pass.
+#include "lq_kernels.hpp"
 #include "lq_plan.hpp"
 
 #include <algorithm>
@@ -935,6 +936,72 @@ bool apply_rotation_scaling(PassPlan &p, bool at_plan_time, int rb, double max_g
 }
 } // namespace
 
+namespace {
+// Tile bits of an operator that runs in a pass of its own, 0 when it does not:
+// its targets and the lowest other bits. Controls stay outside the tile (a
+// tile they rule out is not visited) except on the four low bits, which every
+// tile holds so that HBM is read in runs of 16 amplitudes.
+uint64_t dense_pass_bits(const LOp &o, int n) {
+    if (o.kind != TOP_DENSEK || o.is_dot() || (o.flags & TF_ZERO_UNCTRL) || o.k < 3 || o.k > 6) return 0;
+    uint64_t T = o.target_mask();
+    for (int b = 0; b < n && popc(T) < kDenseTileBits; ++b)
+        if (b < 4 || !((o.cmask >> b) & 1ull)) T |= 1ull << b;
+    return popc(T) == kDenseTileBits ? T : 0;
+}
+
+PassPlan dense_pass(const LOp &o, int index, int n) {
+    PassPlan p;
+    p.dense = true;
+    const uint64_t T = dense_pass_bits(o, n);
+    for (int b = 0; b < n; ++b)
+        if ((T >> b) & 1ull) p.tbits.push_back(b);
+    TileOp t{};
+    t.kind = o.kind;
+    t.flags = o.flags;
+    t.k = static_cast<uint32_t>(o.k);
+    t.smask = o.smask;
+    t.gcmask = o.cmask;
+    t.gcval = o.cval & o.cmask;
+    for (int j = 0; j < o.k; ++j) t.gpos[j] = o.bits[j];
+    p.ops.push_back(t);
+    p.coef = o.coef;
+    for (size_t c = 0; c < o.coef.size(); ++c)
+        p.coef_src.push_back({static_cast<uint32_t>(index), static_cast<uint32_t>(c)});
+    p.load_mask = p.store_mask = o.smask;
+    return p;
+}
+} // namespace
+
+DenseTileArgs dense_tile_args(const PassPlan &p, int n) {
+    LQ_ABORT_IF(!p.dense || p.ops.size() != 1 || p.tbits.size() != kDenseTileBits, "not a dense pass");
+    const TileOp &o = p.ops[0];
+    const int k = static_cast<int>(o.k), cl = kDenseTileBits - k;
+    DenseTileArgs a{};
+    uint64_t T = 0;
+    int col = 0;
+    for (int b = 0; b < kDenseTileBits; ++b) {
+        const int g = p.tbits[b];
+        T |= 1ull << g;
+        a.tb[b] = g;
+        a.lp[b] = -1;
+        for (int j = 0; j < k; ++j)
+            if (o.gpos[j] == g) a.lp[b] = cl + k - 1 - j;
+        if (a.lp[b] >= 0) continue;
+        a.lp[b] = col;
+        if ((o.gcmask >> g) & 1ull) {
+            a.ccmask |= 1u << col;
+            if ((o.gcval >> g) & 1ull) a.ccval |= 1u << col;
+        }
+        ++col;
+    }
+    LQ_ABORT_IF(col != cl, "dense pass targets outside its tile");
+    a.ocval = o.gcval & ~T;
+    for (int b = 0; b < n; ++b)
+        if (!((T >> b) & 1ull) && !((o.gcmask >> b) & 1ull)) a.ob[a.nout++] = b;
+    a.ntiles = 1ull << a.nout;
+    return a;
+}
+
 std::vector<PassPlan> plan_passes(const std::vector<LOp> &ops, const PlanConfig &cfg) {
     const int N = static_cast<int>(ops.size());
     const int n = cfg.n;
@@ -990,6 +1057,10 @@ std::vector<PassPlan> plan_passes(const std::vector<LOp> &ops, const PlanConfig 
     std::set<int> ready;
     for (int j = 0; j < N; ++j)
         if (indeg[j] == 0) ready.insert(j);
+    // operators that run in passes of their own; everything else that is
+    // ready goes first, so they split as few tile passes as possible
+    std::vector<char> alone(N, 0);
+    for (int j = 0; j < N; ++j) alone[j] = cfg.dense_passes && dense_pass_bits(ops[j], n) != 0;
 
     const int ktmax = std::min(cfg.kt_max, n);
     const int low = std::max(0, std::min(cfg.low_bits, ktmax));
@@ -1015,6 +1086,7 @@ std::vector<PassPlan> plan_passes(const std::vector<LOp> &ops, const PlanConfig 
         while (!q.empty()) {
             const int i = q.top();
             q.pop();
+            if (alone[i]) continue;
             if ((nm[i] & ~T) != 0 || (dots >= cfg.max_dots && ops[i].is_dot())) {
                 if (frontier) frontier->push_back(i);
                 continue;
@@ -1068,6 +1140,15 @@ std::vector<PassPlan> plan_passes(const std::vector<LOp> &ops, const PlanConfig 
     std::vector<PassPlan> passes;
     int remaining = N;
     while (remaining > 0) {
+        if (std::all_of(ready.begin(), ready.end(), [&](int i) { return alone[i]; })) {
+            const int i = *ready.begin();
+            ready.erase(ready.begin());
+            --remaining;
+            for (int s : succ[i])
+                if (--indeg[s] == 0) ready.insert(s);
+            passes.push_back(dense_pass(ops[i], i, n));
+            continue;
+        }
         std::vector<int> sel;
         uint64_t T = 0;
         budget = (passes.empty() && cfg.first_budget > 0) ? cfg.first_budget : cfg.budget;
@@ -1080,13 +1161,13 @@ std::vector<PassPlan> plan_passes(const std::vector<LOp> &ops, const PlanConfig 
                 int pick = -1;
                 const bool dots_full = dots >= cfg.max_dots;
                 for (int i : ready)
-                    if ((nm[i] & ~T) == 0 && !(dots_full && ops[i].is_dot())) {
+                    if (!alone[i] && (nm[i] & ~T) == 0 && !(dots_full && ops[i].is_dot())) {
                         pick = i;
                         break;
                     }
                 if (pick < 0)
                     for (int i : ready)
-                        if (popc(T | nm[i]) <= ktmax && !(dots_full && ops[i].is_dot())) {
+                        if (!alone[i] && popc(T | nm[i]) <= ktmax && !(dots_full && ops[i].is_dot())) {
                             pick = i;
                             break;
                         }
@@ -1208,8 +1289,8 @@ std::string plan_structure_key(const std::vector<LOp> &ops, const PlanConfig &cf
     std::string key;
     auto put = [&key](const void *p, size_t n) { key.append(static_cast<const char *>(p), n); };
     const double b = cfg.budget;
-    const int32_t hdr[8] = {cfg.n, cfg.ns, cfg.kt_max, cfg.low_bits, cfg.reg_rb, cfg.max_dots,
-                            cfg.scale_rotations ? 1 : 0, cfg.lookahead ? 1 : 0};
+    const int32_t hdr[9] = {cfg.n, cfg.ns, cfg.kt_max, cfg.low_bits, cfg.reg_rb, cfg.max_dots,
+                            cfg.scale_rotations ? 1 : 0, cfg.lookahead ? 1 : 0, cfg.dense_passes ? 1 : 0};
     put(hdr, sizeof(hdr));
     put(&b, sizeof(b));
     put(&cfg.first_budget, sizeof(cfg.first_budget));

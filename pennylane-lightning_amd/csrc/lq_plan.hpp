@@ -85,6 +85,9 @@ struct PassPlan {
     bool reg = false;
     std::vector<TileStage> stages;
     uint32_t end_transpose = 0;
+    // one dense operator on 3..6 bits in a pass of its own (lq_dense.hip):
+    // tbits are the tile's, ops[0] the operator, coef its matrix
+    bool dense = false;
     // where each coefficient comes from, so a plan can be reused for a
     // program of the same structure with other coefficients: entry i of coef
     // is ops[coef_src[i].op].coef[coef_src[i].idx], or (op == kNoSrc) an
@@ -131,6 +134,9 @@ struct PlanConfig {
     // exceed max_scale_growth keeps every rotation in the full form.
     bool scale_rotations = false;
     double max_scale_growth = 1e300;
+    // dense operators on three to six bits (not dots) run in passes of their
+    // own on the matrix cores instead of as LDS ops of a tile pass
+    bool dense_passes = false;
     // choose each pass's tile bits by lookahead (the bits that let the most
     // work run) instead of taking the first ready op's bits
     bool lookahead = false;
@@ -149,5 +155,9 @@ std::string plan_structure_key(const std::vector<LOp> &ops, const PlanConfig &cf
 bool refresh_plan_coefs(std::vector<PassPlan> &passes, const std::vector<LOp> &ops);
 
 TileGeom make_geom(int n, const std::vector<int> &tbits);
+
+// Launch arguments of a dense pass on n qubits (the states are left to fill in)
+struct DenseTileArgs;
+DenseTileArgs dense_tile_args(const PassPlan &p, int n);
 
 } // namespace lqamd
