@@ -148,6 +148,16 @@ __device__ __forceinline__ unsigned opaque0() {
     asm volatile("" : "+s"(z));
     return z;
 }
+// the first word of the `line`-th 64 bytes of the coefficients, read for the
+// line's way into the L2; keep() is where the load has to have returned
+__device__ __forceinline__ unsigned touch(const double2 *c, const unsigned line, const unsigned lines) {
+    return line < lines ? ((const unsigned *)c)[line * 16u] : 0u;
+}
+__device__ __forceinline__ void keep(const unsigned x) {
+#ifndef LQ_EMU
+    asm volatile("" : : "v"(x));
+#endif
+}
 typedef real nvec __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ cplx ldnt(const cplx *p) {
     const nvec t = __builtin_nontemporal_load(reinterpret_cast<const nvec *>(p));
@@ -255,6 +265,15 @@ class Gen {
         o << "  const unsigned long long bid = (unsigned long long)blockIdx.x + (unsigned long long)blockIdx.y * gridDim.x;\n";
         o << "  if (bid >= ntiles) return;\n";
         o << "  const unsigned long long tile = ntiles >= 8ull ? (bid & 7ull) * (ntiles >> 3) + (bid >> 3) : bid;\n";
+        // the pass's coefficients are used a few at a time through scalar
+        // loads, which miss every cache when the program has just been
+        // uploaded and few workgroups run on an XCD (nothing else brought the
+        // lines in): one touch per 64-byte line, issued before the state's
+        // loads, brings all of them to the XCD's L2 at once (20-qubit circuit,
+        // one tile per CU: 38 -> 29 us a pass; no change at 30 qubits)
+        const size_t lines = (p_.coef.size() + 1) * 16 / 64 + 1;
+        o << "  unsigned tch = 0u;\n";
+        for (size_t l = 0; l < lines; l += 256) o << "  tch |= touch(coef, tid + " << l << "u, " << lines << "u);\n";
         // load straight into the first stage's mapping when its thread
         // bits start with the contiguous low bits (the loads coalesce as
         // in the default mapping): no entry transpose
@@ -283,6 +302,7 @@ class Gen {
             emit_loads("v", "gl0", lm);
         }
         o << "  }\n";
+        o << "  keep(tch);\n";
         emit_tile_body(m0, nslots, lm);
         o << "}\n";
         // the product factors follow the position table
