@@ -121,7 +121,7 @@ bool build_batch_program(int n, int dtype, const OpsList &ops, const Obs &ham, c
     std::vector<uint64_t> tp = tp_in;
     std::sort(tp.begin(), tp.end());
     std::vector<LOp> bwd;
-    if (!tp.empty()) p.scales = backward_sweep(n, ops, tp, 1, 1, bwd);
+    if (!tp.empty()) p.scales = backward_sweep(n, ops, tp, 1, 1, bwd, 0);
     for (const auto &l : bwd)
         if (!to_bop(l, &p, why)) return false;
     p.nslots = 1 + static_cast<uint32_t>(tp.size());

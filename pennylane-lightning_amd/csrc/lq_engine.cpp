@@ -128,20 +128,21 @@ const std::vector<cd> &named_obs_matrix(const std::string &name) {
     LQ_ABORT((std::string("Expval does not exist for named observable ") + name).c_str());
 }
 
-LOp make_dot(LOp op, uint32_t sa, uint32_t sb, int slot) {
-    op.flags = (op.flags & ~TF_ZERO_UNCTRL) | TF_DOT;
+// part: TF_DOT_RE or TF_DOT_IM when only that part of the value is used
+LOp make_dot(LOp op, uint32_t sa, uint32_t sb, int slot, uint32_t part = 0) {
+    op.flags = (op.flags & ~TF_ZERO_UNCTRL) | TF_DOT | part;
     op.sa = sa;
     op.sb = sb;
     op.slot = slot;
     return op;
 }
 
-LOp identity_dot(uint32_t sa, uint32_t sb, int slot) {
+LOp identity_dot(uint32_t sa, uint32_t sb, int slot, uint32_t part = 0) {
     LOp op;
     op.kind = TOP_DIAG;
     op.k = 0;
     op.coef = {1.0};
-    return make_dot(op, sa, sb, slot);
+    return make_dot(op, sa, sb, slot, part);
 }
 
 // Pauli word as the cheapest op form for a dot: a parity op for Z-only
@@ -1428,7 +1429,7 @@ double StateVector::expval_named(const std::string &name, const uint32_t *wires,
     // the pending gates and the dot run as one program
     std::vector<LOp> prog;
     prog.swap(queue_);
-    prog.push_back(make_dot(lower_matrix(m, {phys_bit(n_, wires[0])}, 0, 0, true), 0, 0, 0));
+    prog.push_back(make_dot(lower_matrix(m, {phys_bit(n_, wires[0])}, 0, 0, true), 0, 0, 0, TF_DOT_RE));
     return run(prog, {d_}, 1)[0].real();
 }
 
@@ -1442,7 +1443,7 @@ std::vector<double> StateVector::expval_named_batch(const std::vector<std::strin
         const auto &m = named_obs_matrix(names[i]);
         check_wires(n_, &wires[i], 1, nullptr, 0);
         slot_of[i] = static_cast<int>(dots.size());
-        dots.push_back(make_dot(lower_matrix(m, {phys_bit(n_, wires[i])}, 0, 0, true), 0, 0, slot_of[i]));
+        dots.push_back(make_dot(lower_matrix(m, {phys_bit(n_, wires[i])}, 0, 0, true), 0, 0, slot_of[i], TF_DOT_RE));
     }
     const int nslots = static_cast<int>(dots.size());
     std::vector<LOp> prog;
@@ -1477,7 +1478,7 @@ double StateVector::expval_matrix(const void *mat, const uint32_t *wires, int nw
     }
     std::vector<LOp> prog;
     prog.swap(queue_);
-    prog.push_back(make_dot(lower_matrix(std::move(m), tb, 0, 0, true), 0, 0, 0));
+    prog.push_back(make_dot(lower_matrix(std::move(m), tb, 0, 0, true), 0, 0, 0, TF_DOT_RE));
     return run(prog, {d_}, 1)[0].real();
 }
 
@@ -1915,7 +1916,7 @@ void apply_forward(StateVector &sv, const OpsList &ops, void *state) {
 // trainable parameter change no result and are left out. Returns the
 // generator scales, negated for inverse ops.
 std::vector<double> backward_sweep(int n, const OpsList &ops, const std::vector<uint64_t> &tp, size_t m, int slot0,
-                                   std::vector<LOp> &prog) {
+                                   std::vector<LOp> &prog, uint32_t part) {
     const size_t ntp = tp.size();
     const uint32_t all = (1u << (m + 1)) - 1u;
     std::vector<double> scales(ntp, 0.0);
@@ -1941,7 +1942,7 @@ std::vector<double> backward_sweep(int n, const OpsList &ops, const std::vector<
                 scales[static_cast<size_t>(tnum)] = s * (op.inverse ? -1.0 : 1.0);
                 for (size_t j = 0; j < m; ++j)
                     prog.push_back(make_dot(g, 0, 1 + static_cast<uint32_t>(j),
-                                            slot0 + static_cast<int>(tnum * static_cast<int64_t>(m) + j)));
+                                            slot0 + static_cast<int>(tnum * static_cast<int64_t>(m) + j), part));
                 last_dot = prog.size();
                 --tnum;
                 --tp_pos;
@@ -1995,8 +1996,8 @@ void adjoint_jacobian(StateVector &sv, const OpsList &ops, const std::vector<std
         w.m = m;
         std::vector<LOp> prog;
         if (expvals)
-            for (size_t j = 0; j < m; ++j) prog.push_back(identity_dot(0, 1 + static_cast<uint32_t>(j), w.exp_slots++));
-        w.scales = backward_sweep(sv.n(), ops, tp, m, w.exp_slots, prog);
+            for (size_t j = 0; j < m; ++j) prog.push_back(identity_dot(0, 1 + static_cast<uint32_t>(j), w.exp_slots++, TF_DOT_RE));
+        w.scales = backward_sweep(sv.n(), ops, tp, m, w.exp_slots, prog, TF_DOT_IM);
         w.nslots = w.exp_slots + static_cast<int>(ntp * m);
         w.planned = sv.plan(prog, 1 + static_cast<int>(m));
         return w;
@@ -2064,7 +2065,7 @@ void vector_jacobian_product(StateVector &sv, const OpsList &ops, const void *dy
     if (apply_operations) apply_forward(sv, ops, lam);
     // planned on the host while the forward pass runs
     std::vector<LOp> prog;
-    const std::vector<double> scales = backward_sweep(sv.n(), ops, tp, 1, 0, prog);
+    const std::vector<double> scales = backward_sweep(sv.n(), ops, tp, 1, 0, prog, 0);
     const auto v = sv.execute(sv.plan(prog, 2), {lam, mu}, static_cast<int>(ntp));
     // w_t = i s <G mu | lambda> = i s <mu | G lambda>
     for (size_t t = 0; t < ntp; ++t) out[t] = cd(0.0, scales[t]) * v[t];

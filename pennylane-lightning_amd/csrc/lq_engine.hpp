@@ -381,9 +381,10 @@ LOp lower_record(int n, const OpRec &op, bool dagger);
 // Append the backward sweep on states {lambda, b_1..b_m} to prog: for each
 // trainable op from the last, dots <b_j | G lambda> into slot
 // slot0 + t*m + j, then U^dagger on all states. Returns the generator scales
-// (negated for inverse ops) in sorted-trainable order.
+// (negated for inverse ops) in sorted-trainable order. part: TF_DOT_IM when
+// only the dots' imaginary parts are used, else 0.
 std::vector<double> backward_sweep(int n, const OpsList &ops, const std::vector<uint64_t> &tp, size_t m, int slot0,
-                                   std::vector<LOp> &prog);
+                                   std::vector<LOp> &prog, uint32_t part);
 
 // Backward sweeps run since the last reset (process-wide): shared by a
 // group of observables, and for one observable.

@@ -87,6 +87,12 @@ __device__ __forceinline__ void d1p(cplx &a, cplx &b, const cplx m0, const cplx 
     a = sel(g, x, a);
     b = sel(g, y, b);
 }
+// exchange, where g holds
+__device__ __forceinline__ void swp(cplx &a, cplx &b, const bool g) {
+    const cplx x = sel(g, b, a);
+    b = sel(g, a, b);
+    a = x;
+}
 __device__ __forceinline__ void d2p(cplx &a, cplx &b, cplx &c, cplx &d, const cplx *m, const bool g) {
     cplx w = a, x = b, y = c, z = d;
     d2(w, x, y, z, m);
@@ -170,11 +176,60 @@ __device__ __forceinline__ void stnt(cplx *p, const cplx v) {
     __builtin_nontemporal_store(t, reinterpret_cast<nvec *>(p));
 }
 __device__ __forceinline__ unsigned swz(unsigned l) { return LQ_SWZ; }
-template <int D> __device__ __forceinline__ void dflush(double r, double i, double2 (*dred)[D], unsigned slot) {
-    for (int off = 32; off > 0; off >>= 1) {
-        r += __shfl_xor(r, off, 64);
-        i += __shfl_xor(i, off, 64);
+// dots: r += Re / Im (conj(b) v), and with the sign changed
+__device__ __forceinline__ void are(double &r, const cplx b, const cplx v) { r += (double)b.x * v.x; r += (double)b.y * v.y; }
+__device__ __forceinline__ void aim(double &r, const cplx b, const cplx v) { r += (double)b.x * v.y; r -= (double)b.y * v.x; }
+__device__ __forceinline__ void nre(double &r, const cplx b, const cplx v) { r -= (double)b.x * v.x; r -= (double)b.y * v.y; }
+__device__ __forceinline__ void nim(double &r, const cplx b, const cplx v) { r -= (double)b.x * v.y; r += (double)b.y * v.x; }
+// x summed over the wave, in every lane: steps within rows of 16 lanes by DPP,
+// across rows by row swaps (a shuffle through LDS takes some 100 cycles a step)
+#ifdef LQ_EMU
+__device__ __forceinline__ double wsum(double x) {
+    for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
+    return x;
+}
+#else
+template <int C> __device__ __forceinline__ double dpp(const double x) {
+    int w[2];
+    __builtin_memcpy(w, &x, 8);
+    w[0] = __builtin_amdgcn_mov_dpp(w[0], C, 0xf, 0xf, true);
+    w[1] = __builtin_amdgcn_mov_dpp(w[1], C, 0xf, 0xf, true);
+    double y;
+    __builtin_memcpy(&y, w, 8);
+    return y;
+}
+__device__ __forceinline__ double wsum(double x) {
+    x += dpp<0xB1>(x);  // lanes 1 apart
+    x += dpp<0x4E>(x);  // 2
+    x += dpp<0x141>(x); // the other quad of eight lanes (half row mirrored)
+    x += dpp<0x140>(x); // the other half of the row (row mirrored)
+    unsigned w[2];
+    double y, z;
+    __builtin_memcpy(w, &x, 8);
+    {
+        const auto a = __builtin_amdgcn_permlane16_swap(w[0], w[0], false, false);
+        const auto b = __builtin_amdgcn_permlane16_swap(w[1], w[1], false, false);
+        const unsigned u[2] = {a[0], b[0]}, v[2] = {a[1], b[1]};
+        __builtin_memcpy(&y, u, 8);
+        __builtin_memcpy(&z, v, 8);
+        x = y + z;
     }
+    __builtin_memcpy(w, &x, 8);
+    {
+        const auto a = __builtin_amdgcn_permlane32_swap(w[0], w[0], false, false);
+        const auto b = __builtin_amdgcn_permlane32_swap(w[1], w[1], false, false);
+        const unsigned u[2] = {a[0], b[0]}, v[2] = {a[1], b[1]};
+        __builtin_memcpy(&y, u, 8);
+        __builtin_memcpy(&z, v, 8);
+        x = y + z;
+    }
+    return x;
+}
+#endif
+template <bool R, bool I, int D>
+__device__ __forceinline__ void dflush(double r, double i, double2 (*dred)[D], unsigned slot) {
+    if (R) r = wsum(r);
+    if (I) i = wsum(i);
     if ((threadIdx.x & 63u) == 0) dred[threadIdx.x >> 6][slot] = make_double2(r, i);
 }
 )";
@@ -823,6 +878,31 @@ class Gen {
         const std::string accf = pred ? "accp(" : "acc(";
         const std::string gsuf = pred ? ", gd)" : ")";
         const uint64_t off = t.coef_off;
+        if (dot && (t.flags & (TF_DOT_X | TF_DOT_Y | TF_DOT_Z))) {
+            emit_class_dot(t, A, B, pred);
+            emit_flush(t);
+            o << "  }\n";
+            return;
+        }
+        if ((t.flags & TF_SWAP) && !dot) {
+            // X or SWAP: amplitudes change places, in the registers' names
+            // alone unless a control is a thread bit
+            for (int e = 0; e < E_; ++e) {
+                int e1;
+                if (t.kind == TOP_DENSE1) {
+                    if ((e >> t.lpos[0]) & 1) continue;
+                    e1 = e | (1 << t.lpos[0]);
+                } else {
+                    if (!((e >> t.lpos[0]) & 1) || ((e >> t.lpos[1]) & 1)) continue;
+                    e1 = e ^ (1 << t.lpos[0]) ^ (1 << t.lpos[1]);
+                }
+                if (!elem_ok(t.gcmask, t.gcval, e)) continue;
+                for (int s : sts)
+                    o << "    swp(v" << s << "[" << e << "], v" << s << "[" << e1 << "], " << (pred ? "gd" : "true") << ");\n";
+            }
+            o << "  }\n";
+            return;
+        }
         switch (t.kind) {
         case TOP_DENSE1: {
             const int I = t.lpos[0];
@@ -925,8 +1005,59 @@ class Gen {
         }
         default: LQ_ABORT("kernel generator: unsupported op");
         }
-        if (dot) o << "    dflush(ar, ai, dred, " << t.slot << "u);\n";
+        if (dot) emit_flush(t);
         o << "  }\n";
+    }
+
+    void emit_flush(const TileOp &t) {
+        o_ << "    dflush<" << ((t.flags & TF_DOT_IM) ? "false" : "true") << ", "
+           << ((t.flags & TF_DOT_RE) ? "false" : "true") << ">(ar, ai, dred, " << t.slot << "u);\n";
+    }
+
+    // <b|G|a> for G = X, Y or a diagonal of signs: two multiply-adds per
+    // amplitude and used part instead of a complex product by coefficients
+    // and a complex accumulation
+    void emit_class_dot(const TileOp &t, const std::string &A, const std::string &B, bool pred) {
+        std::ostringstream &o = o_;
+        const bool re = !(t.flags & TF_DOT_IM), im = !(t.flags & TF_DOT_RE);
+        auto el = [](const std::string &v, int e) { return v + "[" + std::to_string(e) + "]"; };
+        if (t.flags & TF_DOT_Z) {
+            // the sign: per element from the register bits, the rest per thread
+            const uint64_t m = t.kind == TOP_PARITY ? t.gpmask : t.k == 0 ? 0ull : 1ull << t.gpos[0];
+            for (int e = 0; e < E_; ++e) {
+                if (!elem_ok(t.gcmask, t.gcval, e)) continue;
+                int neg = 0;
+                for (int i = 0; i < rb_; ++i)
+                    if (((m >> geom_.tb[cur_.r[i]]) & 1ull) && ((e >> i) & 1)) neg ^= 1;
+                const std::string arg = el(B, e) + ", " + el(A, e) + ");\n";
+                if (re) o << "    " << (neg ? "nre" : "are") << "(ar, " << arg;
+                if (im) o << "    " << (neg ? "nim" : "aim") << "(ai, " << arg;
+            }
+            const uint64_t tm = m & ~regmask();
+            if (tm) {
+                o << "    const bool ngt = (pc(gt & " << K(tm) << ") & 1u) != 0u;\n";
+                if (re) o << "    ar = ngt ? -ar : ar;\n";
+                if (im) o << "    ai = ngt ? -ai : ai;\n";
+            }
+        } else {
+            const int I = t.lpos[0];
+            for (int e = 0; e < E_; ++e) {
+                if (((e >> I) & 1) || !elem_ok(t.gcmask, t.gcval, e)) continue;
+                const int e1 = e | (1 << I);
+                const std::string p = el(B, e) + ", " + el(A, e1) + ");\n", q = el(B, e1) + ", " + el(A, e) + ");\n";
+                if (t.flags & TF_DOT_X) {
+                    if (re) o << "    are(ar, " << p << "    are(ar, " << q;
+                    if (im) o << "    aim(ai, " << p << "    aim(ai, " << q;
+                } else { // (Y a)_0 = -i a_1, (Y a)_1 = i a_0
+                    if (re) o << "    aim(ar, " << p << "    nim(ar, " << q;
+                    if (im) o << "    nre(ai, " << p << "    are(ai, " << q;
+                }
+            }
+        }
+        if (pred) {
+            if (re) o << "    ar = gd ? ar : 0.0;\n";
+            if (im) o << "    ai = gd ? ai : 0.0;\n";
+        }
     }
 
     // DIAG (k <= 2 in register passes), PCPHASE, PARITY: a phase per element

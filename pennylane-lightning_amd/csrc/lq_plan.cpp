@@ -70,6 +70,45 @@ uint64_t LOp::dmask() const {
     return m;
 }
 
+bool LOp::is_swap() const {
+    static const cd kX[4] = {0.0, 1.0, 1.0, 0.0};
+    static const cd kSwap[16] = {1.0, 0.0, 0.0, 0.0, 0.0, 0.0, 1.0, 0.0, 0.0, 1.0, 0.0, 0.0, 0.0, 0.0, 0.0, 1.0};
+    if (kind == TOP_DENSE1) return coef.size() == 4 && std::equal(coef.begin(), coef.end(), kX);
+    return kind == TOP_DENSE2 && coef.size() == 16 && std::equal(coef.begin(), coef.end(), kSwap);
+}
+
+uint32_t LOp::dot_class() const {
+    if (!is_dot()) return 0;
+    const cd one(1.0), zero(0.0), im(0.0, 1.0);
+    if (kind == TOP_DENSE1 && coef.size() == 4 && coef[0] == zero && coef[3] == zero) {
+        if (coef[1] == one && coef[2] == one) return TF_DOT_X;
+        if (coef[1] == -im && coef[2] == im) return TF_DOT_Y;
+    }
+    if (((kind == TOP_DIAG && k == 1) || kind == TOP_PARITY) && coef.size() == 2 && coef[0] == one && coef[1] == -one)
+        return TF_DOT_Z;
+    if (kind == TOP_DIAG && k == 0 && coef.size() == 1 && coef[0] == one) return TF_DOT_Z; // no bits: the identity
+    return 0;
+}
+
+bool LOp::is_unitary() const {
+    if (flags & TF_ZERO_UNCTRL) return false;
+    if (kind == TOP_DIAG || kind == TOP_PARITY || kind == TOP_PCPHASE) {
+        for (const cd &v : coef)
+            if (!(std::fabs(std::norm(v) - 1.0) <= 1e-12)) return false;
+        return true;
+    }
+    if (kind != TOP_DENSE1 && kind != TOP_DENSE2) return false;
+    const size_t d = kind == TOP_DENSE1 ? 2 : 4;
+    if (coef.size() != d * d) return false;
+    for (size_t a = 0; a < d; ++a)
+        for (size_t b = a; b < d; ++b) {
+            cd s(a == b ? -1.0 : 0.0);
+            for (size_t r = 0; r < d; ++r) s += std::conj(coef[r * d + a]) * coef[r * d + b];
+            if (!(std::norm(s) <= 1e-24)) return false;
+        }
+    return true;
+}
+
 double LOp::cost() const {
     double c = 0.5;
     switch (kind) {
@@ -295,7 +334,7 @@ void split_1q_rotations(std::vector<LOp> &prog) {
     out.reserve(prog.size() * 3);
     for (auto &o : prog) {
         const bool candidate = (o.kind == TOP_DENSE1 || o.kind == TOP_DENSEK) && o.k == 1 && o.cmask == 0 &&
-                               !o.is_dot() && !(o.flags & TF_ZERO_UNCTRL) && o.coef.size() == 4;
+                               !o.is_dot() && !(o.flags & TF_ZERO_UNCTRL) && o.coef.size() == 4 && !o.is_swap();
         if (!candidate) {
             out.push_back(std::move(o));
             continue;
@@ -340,6 +379,9 @@ void split_1q_rotations(std::vector<LOp> &prog) {
     auto is_phase = [](const LOp &o) {
         return o.kind == TOP_DIAG && o.k == 1 && o.cmask == 0 && !o.is_dot() && o.coef.size() == 2;
     };
+    auto unit_phase = [](const LOp &o) {
+        return std::fabs(std::norm(o.coef[0]) - 1.0) <= 1e-12 && std::fabs(std::norm(o.coef[1]) - 1.0) <= 1e-12;
+    };
     std::vector<char> gone(out.size(), 0);
     for (size_t i = 0; i < out.size(); ++i) {
         if (!is_phase(out[i])) continue;
@@ -348,7 +390,12 @@ void split_1q_rotations(std::vector<LOp> &prog) {
         for (size_t j = i + 1; j < lim; ++j) {
             const LOp &o = out[j];
             if (gone[j]) continue;
-            if (o.is_dot()) break;
+            if (o.is_dot()) {
+                // <b|D^dagger G D|a> = <b|G|a> for a phase on both states and a bit that G acts on diagonally or not at all
+                const uint32_t ab = (1u << o.sa) | (1u << o.sb);
+                if ((out[i].smask & ab) != ab || (o.nmask() & bit) || !unit_phase(out[i])) break;
+                continue;
+            }
             if (!(o.smask & out[i].smask)) continue;
             if (is_phase(o) && o.bits[0] == out[i].bits[0] && o.smask == out[i].smask) {
                 out[j].coef[0] *= out[i].coef[0];
@@ -541,6 +588,32 @@ bool diagonal_kind(uint32_t k) {
 // commute when they act on different states, or when neither acts
 // non-diagonally on a bit the other touches. Dots and ops without a known
 // bit set keep their place relative to everything.
+// Whether a dot (register form, one or two targets) and an op may change
+// places: the op is unitary, acts on both of the dot's states, and acts
+// non-diagonally on no bit the dot touches (and the dot on none of the op's).
+bool dot_commutes(const TileOp &dot, const TileOp &op) {
+    const uint32_t ab = (1u << dot.sa) | (1u << dot.sb);
+    if (!(op.flags & TF_UNITARY) || (op.smask & ab) != ab) return false;
+    auto bits = [](const TileOp &t, uint64_t *nd, uint64_t *dg) {
+        *nd = 0;
+        *dg = t.gcmask;
+        uint64_t m = 0;
+        for (uint32_t j = 0; j < t.k && j < static_cast<uint32_t>(kMaxTileOpTargets); ++j) m |= 1ull << t.gpos[j];
+        switch (t.kind) {
+        case TOP_DENSE1:
+        case TOP_DENSE2: *nd = m; return true;
+        case TOP_DIAG:
+        case TOP_PCPHASE: *dg |= m; return true;
+        case TOP_PARITY: *dg |= t.gpmask; return true;
+        case TOP_SIGN: return true;
+        default: return false;
+        }
+    };
+    uint64_t na, da, nb, db;
+    if (!bits(dot, &na, &da) || !bits(op, &nb, &db)) return false;
+    return !(na & (nb | db)) && !(nb & da);
+}
+
 std::vector<int> stage_levels_order(const std::vector<TileOp> &ops) {
     const int M = static_cast<int>(ops.size());
     const uint64_t ALL = ~0ull;
@@ -566,6 +639,10 @@ std::vector<int> stage_levels_order(const std::vector<TileOp> &ops) {
         dg[x] = d;
     }
     auto commute = [&](int x, int y) {
+        const bool dx = ops[x].flags & TF_DOT, dy = ops[y].flags & TF_DOT;
+        if (dx && dy) return true;
+        if (dx) return dot_commutes(ops[x], ops[y]);
+        if (dy) return dot_commutes(ops[y], ops[x]);
         if (nd[x] == ALL || nd[y] == ALL) return false;
         if (!(ops[x].smask & ops[y].smask)) return true;
         return !(nd[x] & (nd[y] | dg[y])) && !(nd[y] & (nd[x] | dg[x]));
@@ -593,25 +670,39 @@ void group_thread_phases(PassPlan &p, std::vector<TileOp> &ops, const int *ridx)
                t.gpos[0] < 64 && ridx[t.gpos[0]] < 0;
     };
     auto blocker = [&](const TileOp &t) {
-        if (t.flags & TF_DOT) return true;
-        return !diagonal_kind(t.kind) && t.kind != TOP_DENSE1 && t.kind != TOP_DENSE2;
+        return !(t.flags & TF_DOT) && !diagonal_kind(t.kind) && t.kind != TOP_DENSE1 && t.kind != TOP_DENSE2;
     };
     int count = 0;
     for (const TileOp &t : ops) count += is_tphase(t);
     if (count < 2) return;
     std::vector<TileOp> out;
-    std::vector<std::pair<uint32_t, size_t>> open; // (state mask, index into out)
+    struct Group {
+        uint32_t sm;
+        size_t at;      // index into out
+        bool past_dot;  // a dot stands after it
+    };
+    std::vector<Group> open;
     for (const TileOp &t : ops) {
         if (blocker(t)) open.clear();
+        if (t.flags & TF_DOT) {
+            // phases on thread bits commute with a dot whose states they both
+            // act on (its non-diagonal bits are register bits): the group
+            // stays open for unitary ones
+            const uint32_t ab = (1u << t.sa) | (1u << t.sb);
+            open.erase(std::remove_if(open.begin(), open.end(), [&](const Group &g) { return (g.sm & ab) != ab; }),
+                       open.end());
+            for (Group &g : open) g.past_dot = true;
+        }
         if (!is_tphase(t)) {
             out.push_back(t);
             continue;
         }
         size_t at = out.size();
         bool found = false;
-        for (const auto &g : open)
-            if (g.first == t.smask && out[g.second].k < static_cast<uint32_t>(kMaxTileOpTargets)) {
-                at = g.second;
+        for (const Group &g : open)
+            if (g.sm == t.smask && out[g.at].k < static_cast<uint32_t>(kMaxTileOpTargets) &&
+                (!g.past_dot || (t.flags & TF_UNITARY))) {
+                at = g.at;
                 found = true;
             }
         if (!found) {
@@ -625,7 +716,7 @@ void group_thread_phases(PassPlan &p, std::vector<TileOp> &ops, const int *ridx)
             p.coef.insert(p.coef.end(), 2 * kMaxTileOpTargets, cd(1.0));
             p.coef_src.insert(p.coef_src.end(), 2 * kMaxTileOpTargets, PassPlan::CoefSrc{PassPlan::kNoSrc, 0});
             out.push_back(n);
-            open.emplace_back(t.smask, at);
+            open.push_back({t.smask, at, false});
         }
         TileOp &g = out[at];
         const uint64_t dst = g.coef_off + 2 * static_cast<uint64_t>(g.k);
@@ -660,8 +751,16 @@ void group_register_phases(PassPlan &p, int rb) {
                 return t.kind == TOP_DIAG && t.k == 1 && t.gcmask == 0 && !(t.flags & TF_DOT) && t.gpos[0] >= 0 &&
                        t.gpos[0] < 64 && ridx[t.gpos[0]] >= 0;
             };
-            auto blocks = [&](const TileOp &l, int r, uint32_t sm) {
-                if (l.flags & TF_DOT) return true;
+            auto blocks = [&](const TileOp &l, int r, uint32_t sm, bool unit) {
+                if (l.flags & TF_DOT) {
+                    // <b|D^dagger G D|a> = <b|G|a> for a phase D on both states and a
+                    // bit that G acts on diagonally or not at all
+                    const uint32_t ab = (1u << l.sa) | (1u << l.sb);
+                    if (!unit || (sm & ab) != ab) return true;
+                    if (l.kind == TOP_DENSE1) return l.lpos[0] == r;
+                    if (l.kind == TOP_DENSE2) return l.lpos[0] == r || l.lpos[1] == r;
+                    return !diagonal_kind(l.kind);
+                }
                 if (diagonal_kind(l.kind)) return false;
                 if (!(l.smask & sm)) return false;
                 if (l.kind == TOP_DENSE1) return l.lpos[0] == r;
@@ -669,12 +768,12 @@ void group_register_phases(PassPlan &p, int rb) {
                 return true;
             };
             std::vector<TileOp> rest;      // non-phase ops; gap g sits before rest[g]
-            struct Ph { int lo, hi, r; uint32_t sm; cd d0, d1; int at; uint64_t src; };
+            struct Ph { int lo, hi, r; uint32_t sm; cd d0, d1; int at; uint64_t src; bool unit; };
             std::vector<Ph> ph;
             for (const TileOp &t : ops) {
                 if (is_phase(t)) {
                     ph.push_back({0, 0, ridx[t.gpos[0]], t.smask, p.coef[t.coef_off], p.coef[t.coef_off + 1],
-                                  static_cast<int>(rest.size()), t.coef_off});
+                                  static_cast<int>(rest.size()), t.coef_off, (t.flags & TF_UNITARY) != 0});
                 } else {
                     rest.push_back(t);
                 }
@@ -684,9 +783,9 @@ void group_register_phases(PassPlan &p, int rb) {
             std::vector<int> prev_b(ph.size(), -1), next_b(ph.size(), M);
             for (size_t j = 0; j < ph.size(); ++j) {
                 for (int x = ph[j].at - 1; x >= 0; --x)
-                    if (blocks(rest[x], ph[j].r, ph[j].sm)) { prev_b[j] = x; break; }
+                    if (blocks(rest[x], ph[j].r, ph[j].sm, ph[j].unit)) { prev_b[j] = x; break; }
                 for (int x = ph[j].at; x < M; ++x)
-                    if (blocks(rest[x], ph[j].r, ph[j].sm)) { next_b[j] = x; break; }
+                    if (blocks(rest[x], ph[j].r, ph[j].sm, ph[j].unit)) { next_b[j] = x; break; }
             }
             // Reorder the other ops by their earliest level (ops that commute
             // may pass each other), so that ops on different bits at the same
@@ -937,6 +1036,8 @@ bool apply_rotation_scaling(PassPlan &p, bool at_plan_time, int rb, double max_g
 } // namespace
 
 namespace {
+constexpr double kSwapCost = 0.25; // of a 2x2 dense op's 1.0
+
 // Tile bits of an operator that runs in a pass of its own, 0 when it does not:
 // its targets and the lowest other bits. Controls stay outside the tile (a
 // tile they rule out is not visited) except on the four low bits, which every
@@ -1008,6 +1109,7 @@ std::vector<PassPlan> plan_passes(const std::vector<LOp> &ops, const PlanConfig 
     std::vector<std::vector<int>> succ(N);
     std::vector<int> indeg(N, 0), mark(N, -1);
     std::vector<uint64_t> nm(N), dm(N);
+    std::vector<double> cost_of(N);
     struct BitDeps {
         int lastN = -1;
         std::vector<int> D, RN, RD;
@@ -1016,6 +1118,10 @@ std::vector<PassPlan> plan_passes(const std::vector<LOp> &ops, const PlanConfig 
     for (int j = 0; j < N; ++j) {
         nm[j] = ops[j].nmask();
         dm[j] = ops[j].dmask() & ~nm[j];
+        // specialised passes swap the amplitudes of an X or SWAP: a select per
+        // word where a control is a thread bit, nothing otherwise
+        cost_of[j] = ops[j].cost();
+        if (cfg.lookahead && !ops[j].is_dot() && ops[j].is_swap()) cost_of[j] *= kSwapCost / (ops[j].k == 1 ? 1.0 : 2.5);
         LQ_ABORT_IF(((nm[j] | dm[j]) >> n) != 0, "operation acts on a wire outside the state");
         const bool dot = ops[j].is_dot();
         auto dep = [&](int i) {
@@ -1054,6 +1160,7 @@ std::vector<PassPlan> plan_passes(const std::vector<LOp> &ops, const PlanConfig 
         }
     }
 
+    const bool has_dots = std::any_of(ops.begin(), ops.end(), [](const LOp &o) { return o.is_dot(); });
     std::set<int> ready;
     for (int j = 0; j < N; ++j)
         if (indeg[j] == 0) ready.insert(j);
@@ -1091,11 +1198,11 @@ std::vector<PassPlan> plan_passes(const std::vector<LOp> &ops, const PlanConfig 
                 if (frontier) frontier->push_back(i);
                 continue;
             }
-            if (done > 0 && cost + ops[i].cost() > budget) {
+            if (done > 0 && cost + cost_of[i] > budget) {
                 *full = true;
                 break;
             }
-            cost += ops[i].cost();
+            cost += cost_of[i];
             dots += ops[i].is_dot() ? 1 : 0;
             ++done;
             for (int s2 : succ[i]) {
@@ -1172,9 +1279,9 @@ std::vector<PassPlan> plan_passes(const std::vector<LOp> &ops, const PlanConfig 
                             break;
                         }
                 if (pick < 0) break;
-                if (!sel.empty() && cost + ops[pick].cost() > budget) break;
+                if (!sel.empty() && cost + cost_of[pick] > budget) break;
                 T |= nm[pick];
-                cost += ops[pick].cost();
+                cost += cost_of[pick];
                 dots += ops[pick].is_dot() ? 1 : 0;
                 sel.push_back(pick);
                 ready.erase(pick);
@@ -1239,6 +1346,8 @@ std::vector<PassPlan> plan_passes(const std::vector<LOp> &ops, const PlanConfig 
             TileOp t{};
             t.kind = o.kind;
             t.flags = o.flags;
+            if (!o.is_dot() && o.is_swap()) t.flags |= TF_SWAP;
+            if (has_dots) t.flags |= o.is_dot() ? o.dot_class() : o.is_unitary() ? TF_UNITARY : 0u;
             t.k = static_cast<uint32_t>(o.k);
             t.smask = o.smask;
             t.sa = o.sa;
@@ -1296,16 +1405,19 @@ std::string plan_structure_key(const std::vector<LOp> &ops, const PlanConfig &cf
     put(&cfg.first_budget, sizeof(cfg.first_budget));
     put(&cfg.max_scale_growth, sizeof(cfg.max_scale_growth));
     const cd one(1.0), mone(-1.0);
+    const bool has_dots = std::any_of(ops.begin(), ops.end(), [](const LOp &o) { return o.is_dot(); });
     for (const LOp &o : ops) {
         // value tests made while planning (to_register_form)
         uint32_t vflags = 0;
-        if (o.kind == TOP_DENSE1 && (o.flags & TF_REAL) && o.coef.size() == 4 && std::fabs(o.coef[0].real()) < kMinCos)
+        if (!o.is_dot() && o.is_swap()) vflags = 5;
+        else if (o.kind == TOP_DENSE1 && (o.flags & TF_REAL) && o.coef.size() == 4 && std::fabs(o.coef[0].real()) < kMinCos)
             vflags = 4;
         if (o.kind == TOP_DIAG && !o.is_dot()) {
             if (o.k == 1 && o.coef.size() == 2 && o.coef[0] == one && o.coef[1] == mone) vflags = 1;
             else if (o.k == 1 && o.coef.size() == 2 && o.coef[0] == mone && o.coef[1] == one) vflags = 2;
             else if (o.k == 0 && o.coef.size() == 1 && o.coef[0] == mone) vflags = 3;
         }
+        if (has_dots) vflags |= o.is_dot() ? o.dot_class() : o.is_unitary() ? TF_UNITARY : 0u;
         const uint32_t w[8] = {o.kind, o.flags, static_cast<uint32_t>(o.k), o.smask, o.sa, o.sb,
                                static_cast<uint32_t>(o.slot), vflags};
         put(w, sizeof(w));

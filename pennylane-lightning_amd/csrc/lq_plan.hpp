@@ -35,6 +35,12 @@ struct LOp {
     // bits acted on diagonally (controls, diagonal targets, Z parts)
     uint64_t dmask() const;
     double cost() const;
+    // a 2x2 X or 4x4 SWAP (on any targets, with any controls), exactly
+    bool is_swap() const;
+    // TF_DOT_X / TF_DOT_Y / TF_DOT_Z of a dot's operator, or 0
+    uint32_t dot_class() const;
+    // U^dagger U = 1 (of the operator on its targets) to 1e-12
+    bool is_unitary() const;
 };
 
 inline int phys_bit(int n, uint32_t wire) { return n - 1 - static_cast<int>(wire); }

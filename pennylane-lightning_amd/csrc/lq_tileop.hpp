@@ -63,6 +63,13 @@ enum TileOpFlags : uint32_t {
     TF_ZERO_UNCTRL = 2u, // zero the amplitudes outside the control subspace (generators)
     TF_REAL = 4u,        // dense op with real coefficients (imaginary parts zero)
     TF_SCALED = 8u,      // real rotation stored as [[1, -t], [t, 1]]; its cosine is applied once per pass
+    TF_SWAP = 16u,       // the matrix is exactly X (DENSE1) or SWAP (DENSE2): amplitudes change places
+    TF_DOT_X = 32u,      // dot operators with one class of matrix (at most one flag): X,
+    TF_DOT_Y = 64u,      // Y,
+    TF_DOT_Z = 128u,     // diag(1, -1) on a bit or a parity (no bits: the identity)
+    TF_DOT_RE = 256u,    // only the real part of the dot is used
+    TF_DOT_IM = 512u,    // only the imaginary part is used
+    TF_UNITARY = 1024u,  // planning: applied to every state of a dot it commutes with, it leaves the dot unchanged
 };
 
 struct alignas(16) TileOp {
