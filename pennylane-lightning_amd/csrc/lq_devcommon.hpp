@@ -4,6 +4,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <cstddef>
+
 #include "lq_tileop.hpp"
 
 namespace lqamd {
@@ -71,12 +73,110 @@ template <int ELEM_BYTES> __device__ __forceinline__ uint32_t swz(uint32_t l) {
     return l ^ (((l >> 4) ^ (l >> 8)) & 15u);
 }
 
-// Wave-level sum of (re, im) into lane 0.
-__device__ __forceinline__ void wave_sum(double &re, double &im) {
-    for (int off = 32; off > 0; off >>= 1) {
-        re += __shfl_xor(re, off, 64);
-        im += __shfl_xor(im, off, 64);
+template <int CTRL> __device__ __forceinline__ double dpp_mov(double x) {
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(x), CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(x), CTRL, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+// x summed over the 64 lanes, in every lane: within rows of 16 lanes by DPP,
+// across rows by row swaps. (Six shuffles through LDS were some 100 cycles
+// each, most of a dot's time in passes of a few workgroups.)
+__device__ __forceinline__ double wave_sum1(double x) {
+    x += dpp_mov<0xB1>(x);  // lanes 1 apart
+    x += dpp_mov<0x4E>(x);  // 2
+    x += dpp_mov<0x141>(x); // the other quad of eight lanes (half row mirrored)
+    x += dpp_mov<0x140>(x); // the other half of the row (row mirrored)
+    {
+        const auto l = __builtin_amdgcn_permlane16_swap(__double2loint(x), __double2loint(x), false, false);
+        const auto h = __builtin_amdgcn_permlane16_swap(__double2hiint(x), __double2hiint(x), false, false);
+        x = __hiloint2double(h[0], l[0]) + __hiloint2double(h[1], l[1]);
     }
+    const auto l = __builtin_amdgcn_permlane32_swap(__double2loint(x), __double2loint(x), false, false);
+    const auto h = __builtin_amdgcn_permlane32_swap(__double2hiint(x), __double2hiint(x), false, false);
+    return __hiloint2double(h[0], l[0]) + __hiloint2double(h[1], l[1]);
+}
+// Wave-level sum of (re, im).
+__device__ __forceinline__ void wave_sum(double &re, double &im) {
+    re = wave_sum1(re);
+    im = wave_sum1(im);
+}
+
+// Bring `bytes` of a pass's program (op heads, stages) to the XCD's L2 and the
+// CU's cache, one touch per 64-byte line by the workgroup's threads: after an
+// upload, and where one workgroup runs on a CU, each line would otherwise come
+// from HBM when the op that it belongs to is next.
+__device__ __forceinline__ void warm_program(const void *p, uint32_t bytes) {
+    unsigned x = 0;
+    for (uint32_t o = threadIdx.x * 64u; o < bytes; o += kBlock * 64u)
+        x |= *reinterpret_cast<const unsigned *>(static_cast<const char *>(p) + o);
+    asm volatile("" : : "v"(x));
+}
+
+// An op's head held across the wave, word i in lane i of one register: a field
+// is one readlane where it is used. (Scalar loads of the fields were five or
+// six dependent round trips per op; whole heads in scalar registers, the next
+// one's beside the current one's, spilled.)
+struct OpView {
+    uint32_t w;
+    static __device__ __forceinline__ OpView load(const OpHead *h) {
+        const uint32_t lane = threadIdx.x & 63u;
+        constexpr uint32_t kWords = sizeof(OpHead) / 4;
+        return OpView{reinterpret_cast<const uint32_t *>(h)[lane < kWords ? lane : 0u]};
+    }
+    __device__ __forceinline__ uint32_t u32(int i) const { return __builtin_amdgcn_readlane(w, i); }
+    __device__ __forceinline__ uint64_t u64(int i) const { return u32(i) | (static_cast<uint64_t>(u32(i + 1)) << 32); }
+    __device__ __forceinline__ double f64(int i) const { return __hiloint2double(u32(i + 1), u32(i)); }
+    __device__ __forceinline__ uint32_t kind() const { return u32(0); }
+    __device__ __forceinline__ uint32_t flags() const { return u32(1); }
+    __device__ __forceinline__ uint32_t k() const { return u32(2); }
+    __device__ __forceinline__ uint32_t smask() const { return u32(3); }
+    __device__ __forceinline__ uint32_t sa() const { return u32(4); }
+    __device__ __forceinline__ uint32_t sb() const { return u32(5); }
+    __device__ __forceinline__ uint32_t slot() const { return u32(6); }
+    __device__ __forceinline__ uint32_t nz() const { return u32(7); }
+    __device__ __forceinline__ uint32_t lcmask() const { return u32(8); }
+    __device__ __forceinline__ uint32_t lcval() const { return u32(9); }
+    __device__ __forceinline__ uint32_t lxmask() const { return u32(10); }
+    __device__ __forceinline__ uint32_t lzmask() const { return u32(11); }
+    __device__ __forceinline__ int lp0() const { return static_cast<int>(u32(12)); }
+    __device__ __forceinline__ int lp1() const { return static_cast<int>(u32(13)); }
+    __device__ __forceinline__ int gp0() const { return static_cast<int>(u32(14)); }
+    __device__ __forceinline__ int gp1() const { return static_cast<int>(u32(15)); }
+    __device__ __forceinline__ uint64_t ocmask() const { return u64(16); }
+    __device__ __forceinline__ uint64_t ocval() const { return u64(18); }
+    __device__ __forceinline__ uint64_t omask() const { return u64(20); }
+    __device__ __forceinline__ uint64_t gcmask() const { return u64(22); }
+    __device__ __forceinline__ uint64_t gcval() const { return u64(24); }
+    __device__ __forceinline__ uint64_t gpmask() const { return u64(26); }
+    __device__ __forceinline__ uint64_t coef_off() const { return u64(28); }
+    __device__ __forceinline__ uint64_t pc_dim() const { return u64(30); }
+    // coefficient i < 4
+    template <typename T> __device__ __forceinline__ typename VecT<T>::type c(int i) const {
+        return mk<T>(static_cast<T>(f64(32 + 4 * i)), static_cast<T>(f64(34 + 4 * i)));
+    }
+};
+static_assert(offsetof(OpHead, lp0) == 48 && offsetof(OpHead, ocmask) == 64 && offsetof(OpHead, pc_dim) == 120 &&
+                  offsetof(OpHead, c) == 128 && sizeof(OpHead) == 192,
+              "OpView's word numbers");
+
+// bits of x (bit j -> position pos[j]); pos is a kernel argument whose entries
+// come eight to a scalar load, not one load and wait per bit
+template <int MAX> __device__ __forceinline__ uint64_t deposit_bits(uint64_t x, const int32_t (&pos)[MAX], int cnt) {
+    uint64_t r = 0;
+    for (int j = 0; j < cnt; j += 8) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            if (j + u < cnt) r |= ((x >> (j + u)) & 1ull) << pos[j + u];
+    }
+    return r;
+}
+// the offset of tile-local index l: its bits at the tile's positions (entries
+// past the tile's bits meet zero bits of l)
+template <int MAX> __device__ __forceinline__ uint64_t spread_bits(uint32_t l, const int32_t (&tb)[MAX]) {
+    uint64_t r = 0;
+#pragma unroll
+    for (int b = 0; b < 13; ++b) r |= static_cast<uint64_t>((l >> b) & 1u) << tb[b];
+    return r;
 }
 
 // One op on the LDS copy of a tile (kt tile-local bits, tsize = 2^kt). Gate
@@ -85,26 +185,26 @@ __device__ __forceinline__ void wave_sum(double &re, double &im) {
 // the caller places the barrier after it. With SWZ, LDS holds element l at
 // swz(l).
 template <typename T, int NS, bool SWZ>
-__device__ void lds_apply_op(const TileOp &op, typename VecT<T>::type *lds, uint32_t tsize, uint64_t base,
+__device__ void lds_apply_op(const OpView &op, const TileOp &tail, typename VecT<T>::type *lds, uint32_t tsize, uint64_t base,
                              const double2 *coef, double &accr, double &acci) {
     using V = typename VecT<T>::type;
     constexpr int EB = sizeof(V);
     auto at = [](uint32_t l) -> uint32_t { return SWZ ? swz<EB>(l) : l; };
     const uint32_t tid = threadIdx.x;
-    const uint32_t kind = op.kind;
-    const bool dot = (op.flags & TF_DOT) != 0;
-    const bool zero_unctrl = (op.flags & TF_ZERO_UNCTRL) != 0;
-    const uint32_t smask = op.smask;
-    const uint32_t lcm = op.lcmask, lcv = op.lcval;
+    const uint32_t kind = op.kind();
+    const bool dot = (op.flags() & TF_DOT) != 0;
+    const bool zero_unctrl = (op.flags() & TF_ZERO_UNCTRL) != 0;
+    const uint32_t smask = op.smask();
+    const uint32_t lcm = op.lcmask(), lcv = op.lcval();
     const V zero = mk<T>(T(0), T(0));
-    const V *A = lds + op.sa * tsize;
-    const V *B = lds + op.sb * tsize;
+    const V *A = lds + op.sa() * tsize;
+    const V *B = lds + op.sb() * tsize;
 
     if (kind == TOP_DENSE1) {
-        const int q = op.lpos[0];
+        const int q = op.lp0();
         const uint32_t qb = 1u << q;
-        const V m00 = ld_coef<T>(coef, op.coef_off + 0), m01 = ld_coef<T>(coef, op.coef_off + 1);
-        const V m10 = ld_coef<T>(coef, op.coef_off + 2), m11 = ld_coef<T>(coef, op.coef_off + 3);
+        const V m00 = op.template c<T>(0), m01 = op.template c<T>(1);
+        const V m10 = op.template c<T>(2), m11 = op.template c<T>(3);
         for (uint32_t p = tid; p < (tsize >> 1); p += kBlock) {
             const uint32_t i0 = insert_zero(p, q), i1 = i0 | qb;
             const uint32_t j0 = at(i0), j1 = at(i1);
@@ -132,12 +232,12 @@ __device__ void lds_apply_op(const TileOp &op, typename VecT<T>::type *lds, uint
             }
         }
     } else if (kind == TOP_DENSE2) {
-        const int q0 = op.lpos[0], q1 = op.lpos[1];
+        const int q0 = op.lp0(), q1 = op.lp1();
         const int lo = q0 < q1 ? q0 : q1, hi = q0 < q1 ? q1 : q0;
         const uint32_t b0 = 1u << q0, b1 = 1u << q1;
         V m[16];
 #pragma unroll
-        for (int e = 0; e < 16; ++e) m[e] = ld_coef<T>(coef, op.coef_off + e);
+        for (int e = 0; e < 16; ++e) m[e] = ld_coef<T>(coef, op.coef_off() + e);
         for (uint32_t p = tid; p < (tsize >> 2); p += kBlock) {
             const uint32_t i00 = insert_zero(insert_zero(p, lo), hi);
             const uint32_t idx[4] = {at(i00), at(i00 | b1), at(i00 | b0), at(i00 | b0 | b1)};
@@ -177,10 +277,10 @@ __device__ void lds_apply_op(const TileOp &op, typename VecT<T>::type *lds, uint
             }
         }
     } else if (kind == TOP_DENSEK) {
-        const int k = static_cast<int>(op.k);
+        const int k = static_cast<int>(op.k());
         const uint32_t dim = 1u << k;
         int srt[kMaxTileOpTargets];
-        for (int j = 0; j < k; ++j) srt[j] = op.lpos[j];
+        for (int j = 0; j < k; ++j) srt[j] = tail.lpos[j];
         for (int i = 1; i < k; ++i)
             for (int j = i; j > 0 && srt[j - 1] > srt[j]; --j) {
                 const int t = srt[j];
@@ -189,13 +289,13 @@ __device__ void lds_apply_op(const TileOp &op, typename VecT<T>::type *lds, uint
             }
         auto lsp = [&](uint32_t col) -> uint32_t {
             uint32_t o = 0;
-            for (int j = 0; j < k; ++j) o |= ((col >> (k - 1 - j)) & 1u) << op.lpos[j];
+            for (int j = 0; j < k; ++j) o |= ((col >> (k - 1 - j)) & 1u) << tail.lpos[j];
             return o;
         };
         const uint32_t R = dim > static_cast<uint32_t>(kBlock) ? dim / kBlock : 1u;
         const uint32_t per_round = kBlock * R;
         const uint32_t rounds = tsize > per_round ? tsize / per_round : 1u;
-        const double2 *M = coef + op.coef_off;
+        const double2 *M = coef + op.coef_off();
         for (int s = 0; s < (dot ? 1 : NS); ++s) {
             if (!dot && !((smask >> s) & 1u)) continue;
             V *S = dot ? const_cast<V *>(A) : lds + s * tsize;
@@ -241,22 +341,29 @@ __device__ void lds_apply_op(const TileOp &op, typename VecT<T>::type *lds, uint
             }
         }
     } else if (kind == TOP_DIAG || kind == TOP_PCPHASE) {
-        const int k = static_cast<int>(op.k);
+        const int k = static_cast<int>(op.k());
+        auto lpos = [&](int j) { return j == 0 ? op.lp0() : j == 1 ? op.lp1() : tail.lpos[j]; };
+        auto gpos = [&](int j) { return j == 0 ? op.gp0() : j == 1 ? op.gp1() : tail.gpos[j]; };
         uint32_t idx_out = 0;
         for (int j = 0; j < k; ++j)
-            if (op.lpos[j] < 0) idx_out |= static_cast<uint32_t>((base >> op.gpos[j]) & 1ull) << (k - 1 - j);
-        const double2 *D = coef + op.coef_off;
+            if (lpos(j) < 0) idx_out |= static_cast<uint32_t>((base >> gpos(j)) & 1ull) << (k - 1 - j);
+        const double2 *D = coef + op.coef_off();
         // DIAG k=0 holds one entry; only PCPHASE has a second one
-        const V d0 = ld_coef<T>(D, 0);
-        const V d1 = (kind == TOP_PCPHASE) ? ld_coef<T>(D, 1) : d0;
+        const V d0 = op.template c<T>(0), d1 = op.template c<T>(1), d2 = op.template c<T>(2), d3 = op.template c<T>(3);
         for (uint32_t l = tid; l < tsize; l += kBlock) {
             const bool ok = (l & lcm) == lcv;
             uint32_t idx = idx_out;
             for (int j = 0; j < k; ++j)
-                if (op.lpos[j] >= 0) idx |= ((l >> op.lpos[j]) & 1u) << (k - 1 - j);
+                if (lpos(j) >= 0) idx |= ((l >> lpos(j)) & 1u) << (k - 1 - j);
             V d;
-            if (kind == TOP_PCPHASE) d = (idx < op.pc_dim) ? d0 : d1;
-            else d = (k == 0) ? d0 : ld_coef<T>(D, idx);
+            if (kind == TOP_PCPHASE) {
+                d = (idx < op.pc_dim()) ? d0 : d1;
+            } else if (k <= 2) {
+                const V d01 = (idx & 1u) ? d1 : d0, d23 = (idx & 1u) ? d3 : d2;
+                d = (idx & 2u) ? d23 : d01;
+            } else {
+                d = ld_coef<T>(D, idx);
+            }
             const uint32_t j = at(l);
             if (dot) {
                 if (ok) acc_dot(accr, acci, B[j], cmul(d, A[j]));
@@ -271,11 +378,11 @@ __device__ void lds_apply_op(const TileOp &op, typename VecT<T>::type *lds, uint
             }
         }
     } else if (kind == TOP_PARITY) {
-        const uint32_t pout = __popcll(base & op.omask) & 1u;
-        const V d0 = ld_coef<T>(coef, op.coef_off), d1 = ld_coef<T>(coef, op.coef_off + 1);
+        const uint32_t pout = __popcll(base & op.omask()) & 1u;
+        const V d0 = op.template c<T>(0), d1 = op.template c<T>(1);
         for (uint32_t l = tid; l < tsize; l += kBlock) {
             const bool ok = (l & lcm) == lcv;
-            const uint32_t par = (__popc(l & op.lxmask) & 1u) ^ pout;
+            const uint32_t par = (__popc(l & op.lxmask()) & 1u) ^ pout;
             const V d = par ? d1 : d0;
             const uint32_t j = at(l);
             if (dot) {
@@ -291,9 +398,9 @@ __device__ void lds_apply_op(const TileOp &op, typename VecT<T>::type *lds, uint
             }
         }
     } else if (kind == TOP_PAULI) {
-        const uint32_t lx = op.lxmask, lz = op.lzmask;
-        const uint32_t sout = __popcll(base & op.omask) & 1u;
-        const V cp = ld_coef<T>(coef, op.coef_off);
+        const uint32_t lx = op.lxmask(), lz = op.lzmask();
+        const uint32_t sout = __popcll(base & op.omask()) & 1u;
+        const V cp = op.template c<T>(0);
         const V cm = cneg(cp);
         if (dot) {
             for (uint32_t l = tid; l < tsize; l += kBlock) {

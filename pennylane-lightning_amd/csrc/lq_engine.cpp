@@ -723,6 +723,8 @@ StateVector::Planned StateVector::plan(const std::vector<LOp> &prog, int ns, boo
     cfg.low_bits = t.low_bits >= 0 ? t.low_bits : (dtype_ ? 4 : 5);
     cfg.budget = t.budget > 0 ? t.budget : 24.0;
     cfg.dense_passes = true;
+    // a state that is one tile gains nothing from a second pass
+    if (t.budget <= 0 && n_ <= cfg.kt_max) cfg.budget = 1e9;
     // register-resident passes for tiles of 11 or 12 bits with one or two states
     const int ktr = std::min(cfg.kt_max, 8 + kMaxRegBits);
     if (t.reg && ns <= 2 && n_ >= 11 && ktr >= 11) {
@@ -835,6 +837,44 @@ StateVector::Planned StateVector::plan(const std::vector<LOp> &prog, int ns, boo
     return out;
 }
 
+namespace {
+void fill_heads(OpHead *h, const PassPlan &p) {
+    for (size_t i = 0; i < p.ops.size(); ++i) {
+        const TileOp &t = p.ops[i];
+        OpHead o{};
+        o.kind = t.kind;
+        o.flags = t.flags;
+        o.k = t.k;
+        o.smask = t.smask;
+        o.sa = t.sa;
+        o.sb = t.sb;
+        o.slot = t.slot;
+        o.nz = t.nz;
+        o.lcmask = t.lcmask;
+        o.lcval = t.lcval;
+        o.lxmask = t.lxmask;
+        o.lzmask = t.lzmask;
+        o.lp0 = t.lpos[0];
+        o.lp1 = t.lpos[1];
+        o.gp0 = t.gpos[0];
+        o.gp1 = t.gpos[1];
+        o.ocmask = t.ocmask;
+        o.ocval = t.ocval;
+        o.omask = t.omask;
+        o.gcmask = t.gcmask;
+        o.gcval = t.gcval;
+        o.gpmask = t.gpmask;
+        o.coef_off = t.coef_off;
+        o.pc_dim = t.pc_dim;
+        for (size_t c = 0; c < 4 && t.coef_off + c < p.coef.size(); ++c) {
+            o.c[2 * c] = p.coef[t.coef_off + c].real();
+            o.c[2 * c + 1] = p.coef[t.coef_off + c].imag();
+        }
+        h[i] = o;
+    }
+}
+} // namespace
+
 StateVector::Pending StateVector::profile_begin(const PassPlan &pp, double states, bool specialised) {
     Pending pe{};
     pe.a = take_event();
@@ -864,16 +904,22 @@ std::vector<cd> StateVector::execute(const Planned &pl, const std::vector<void *
     if (passes.empty()) return result;
 
     auto align = [](size_t x) { return (x + 255) & ~static_cast<size_t>(255); };
-    std::vector<size_t> op_off(passes.size()), coef_off(passes.size()), part_off(passes.size()),
+    std::vector<size_t> op_off(passes.size()), head_off(passes.size()), coef_off(passes.size()), part_off(passes.size()),
         st_off(passes.size()), geo_slots(passes.size(), 0);
-    size_t ops_bytes = 0, coef_n = 0, part_n = 0, st_bytes = 0;
+    // specialised and dense passes read their coefficients only
+    auto interpreted = [&](size_t p) { return !fns[p] && !passes[p].dense; };
+    size_t heads_bytes = 0, ops_bytes = 0, coef_n = 0, part_n = 0, st_bytes = 0;
     std::vector<SlotRange> ranges(static_cast<size_t>(nslots), SlotRange{0, 0});
     std::vector<char> seen(static_cast<size_t>(nslots), 0);
     for (size_t p = 0; p < passes.size(); ++p) {
+        head_off[p] = heads_bytes;
         op_off[p] = ops_bytes;
-        ops_bytes += passes[p].ops.size() * sizeof(TileOp);
         st_off[p] = st_bytes;
-        st_bytes += passes[p].stages.size() * sizeof(TileStage);
+        if (interpreted(p)) {
+            heads_bytes += passes[p].ops.size() * sizeof(OpHead);
+            ops_bytes += passes[p].ops.size() * sizeof(TileOp);
+            st_bytes += passes[p].stages.size() * sizeof(TileStage);
+        }
         coef_off[p] = coef_n;
         // + the deferred-preparation marker, the specialised kernel's table of
         // bit positions (two per entry) and the product factors read by
@@ -890,7 +936,8 @@ std::vector<cd> StateVector::execute(const Planned &pl, const std::vector<void *
         }
         part_n += passes[p].slot_ids.size() * ntiles;
     }
-    const size_t stages_at = align(ops_bytes);
+    const size_t ops_at = align(heads_bytes);
+    const size_t stages_at = align(ops_at + ops_bytes);
     const size_t coef_at = align(stages_at + st_bytes);
     const size_t ranges_at = align(coef_at + coef_n * sizeof(double2));
     const size_t total = align(ranges_at + ranges.size() * sizeof(SlotRange));
@@ -919,8 +966,11 @@ std::vector<cd> StateVector::execute(const Planned &pl, const std::vector<void *
     stg.ensure(total);
     char *hs = static_cast<char *>(stg.p);
     for (size_t p = 0; p < passes.size(); ++p) {
-        std::memcpy(hs + op_off[p], passes[p].ops.data(), passes[p].ops.size() * sizeof(TileOp));
-        if (!passes[p].stages.empty())
+        if (interpreted(p)) {
+            fill_heads(reinterpret_cast<OpHead *>(hs + head_off[p]), passes[p]);
+            std::memcpy(hs + ops_at + op_off[p], passes[p].ops.data(), passes[p].ops.size() * sizeof(TileOp));
+        }
+        if (interpreted(p) && !passes[p].stages.empty())
             std::memcpy(hs + stages_at + st_off[p], passes[p].stages.data(), passes[p].stages.size() * sizeof(TileStage));
         double2 *c = reinterpret_cast<double2 *>(hs + coef_at) + coef_off[p];
         for (size_t i = 0; i < passes[p].coef.size(); ++i)
@@ -953,6 +1003,7 @@ std::vector<cd> StateVector::execute(const Planned &pl, const std::vector<void *
     if (capturing_) {
         capturing_->coef_at = coef_at;
         capturing_->coef_off = coef_off;
+        capturing_->head_off = head_off;
     }
     const bool prof = prof_ && !capturing_;
 
@@ -976,7 +1027,8 @@ std::vector<cd> StateVector::execute(const Planned &pl, const std::vector<void *
         }
         TilePassArgs a{};
         for (int s = 0; s < ns; ++s) a.sv[s] = states[s];
-        a.ops = reinterpret_cast<const TileOp *>(dp + op_off[p]);
+        a.heads = reinterpret_cast<const OpHead *>(dp + head_off[p]);
+        a.ops = reinterpret_cast<const TileOp *>(dp + ops_at + op_off[p]);
         a.coef = reinterpret_cast<const double2 *>(dp + coef_at) + coef_off[p];
         a.partials = static_cast<double2 *>(partials_.p) + part_off[p];
         a.nops = static_cast<uint32_t>(pp.ops.size());
@@ -993,10 +1045,12 @@ std::vector<cd> StateVector::execute(const Planned &pl, const std::vector<void *
             LQ_ABORT_IF(pp.slot_ids.size() > static_cast<size_t>(fns[p] && ns > 2 ? kMaxJitPassDots : kMaxPassDots),
                         "too many dots in one pass");
             for (int s = 0; s < ns; ++s) ra.sv[s] = states[s];
+            ra.heads = a.heads;
             ra.ops = a.ops;
             ra.stages = reinterpret_cast<const TileStage *>(dp + stages_at + st_off[p]);
             ra.coef = a.coef;
             ra.partials = a.partials;
+            ra.nops = a.nops;
             ra.nstages = static_cast<uint32_t>(pp.stages.size());
             ra.nslots = static_cast<uint32_t>(pp.slot_ids.size());
             ra.load_mask = pp.load_mask;
@@ -1154,6 +1208,7 @@ void StateVector::replay(Recording &r, const double *params, size_t np) {
         double2 *c = reinterpret_cast<double2 *>(hs + r.coef_at) + r.coef_off[p];
         const std::vector<cd> &cf = pl.passes[p].coef;
         for (size_t i = 0; i < cf.size(); ++i) c[i] = make_double2(cf[i].real(), cf[i].imag());
+        if (!pl.fns[p] && !pl.passes[p].dense) fill_heads(reinterpret_cast<OpHead *>(hs + r.head_off[p]), pl.passes[p]);
     }
     hip_check(hipGraphLaunch(r.exec, stream_), "hipGraphLaunch");
     ++r.replays;
@@ -1597,9 +1652,14 @@ double StateVector::expval_obs(const Obs &o) {
     }
     std::vector<PauliWord> words;
     const bool pauli = obs_to_pauli(o, n_, &words);
-    const int ktm = std::min(kt_for(1), n_);
-    bool fits = pauli && words.size() <= 32;
-    for (const auto &w : words) fits = fits && __builtin_popcountll(w.x) <= ktm - 2;
+    // Words that are dots of register passes (diagonal ones, and those on one
+    // or two wires) run in one program with the pending gates, up to the dots
+    // of one pass. Longer words would be LDS dots of generic passes, some
+    // 25 us for seven of them on 15 qubits (four passes for 30 words) against
+    // 3 us for the whole sum in the Pauli-sum kernel, and on large states a
+    // generic pass costs several reads of the state.
+    bool fits = pauli && words.size() <= static_cast<size_t>(kMaxPassDots);
+    for (const auto &w : words) fits = fits && (w.x == 0 || __builtin_popcountll(w.x | w.yz) <= 2);
     if (!fits) flush();
     if (pauli) {
         if (fits) {

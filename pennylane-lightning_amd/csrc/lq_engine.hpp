@@ -260,7 +260,7 @@ class StateVector {
         size_t nparams = 0;
         Planned planned;
         size_t coef_at = 0;
-        std::vector<size_t> coef_off;
+        std::vector<size_t> coef_off, head_off;
         HostPinned staging;
         DevBuf prog;
         hipGraph_t graph = nullptr;

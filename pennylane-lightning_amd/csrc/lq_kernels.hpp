@@ -11,9 +11,14 @@
 
 namespace lqamd {
 
+// Up to this many workgroups a launch brings its program to the caches before
+// it interprets it; larger launches find it there after their first tiles.
+constexpr uint64_t kWarmTiles = 1024;
+
 struct TilePassArgs {
     void *sv[kMaxStates];     // state base pointers (complex<T>)
-    const TileOp *ops;        // device program for this pass
+    const OpHead *heads;      // device program for this pass
+    const TileOp *ops;
     const double2 *coef;      // device coefficient buffer (complex double)
     double2 *partials;        // dot partial sums: [slot][tile], slots local to the pass
     uint32_t nops;
@@ -42,10 +47,12 @@ template <typename T> void launch_tile_pass(const TilePassArgs &a, size_t lds_by
 // one or two states.
 struct TileRegArgs {
     void *sv[kMaxStates]; // the generic kernel takes two; specialised passes up to four
+    const OpHead *heads;
     const TileOp *ops;
     const TileStage *stages;
     const double2 *coef;
     double2 *partials;        // [slot][tile]
+    uint32_t nops;
     uint32_t nstages;
     uint32_t nslots;          // dot slots of the pass (<= kMaxPassDots)
     uint32_t load_mask;

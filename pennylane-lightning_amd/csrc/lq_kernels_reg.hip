@@ -9,8 +9,10 @@
 // between stages is one LDS transpose (XOR-swizzled addresses). Loads and
 // stores use the mapping "thread bits = tile bits 0..7", whose low tile bits
 // are contiguous in HBM, so a wave reads and writes runs of consecutive
-// amplitudes. Dot products (expvals, adjoint generator terms) are reduced per
-// wave into LDS and written once per tile.
+// amplitudes. Launches of few tiles are bound by the latency of the program:
+// heads are brought to the caches first and read one op ahead (13 qubits, two
+// states: 41-47 us -> 28 us a pass). Dot products (expvals, adjoint generator
+// terms) are reduced per wave into LDS and written once per tile.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -66,11 +68,11 @@ template <int NS, typename F> __device__ __forceinline__ void with_pair(uint32_t
 
 // One-bit phase diag(d0, d1), no controls, on register bit I of the stage.
 template <typename T, int NS, int RB, int I>
-__device__ __forceinline__ void reg_phase_reg(Regs<T, NS, RB> &R, const TileOp &op, typename VecT<T>::type d0,
+__device__ __forceinline__ void reg_phase_reg(Regs<T, NS, RB> &R, const OpView &op, typename VecT<T>::type d0,
                                               typename VecT<T>::type d1, double &accr, double &acci) {
     constexpr int E = 1 << RB;
-    if (op.flags & TF_DOT) {
-        with_pair<NS>(op.sa, op.sb, [&](auto A, auto B) {
+    if (op.flags() & TF_DOT) {
+        with_pair<NS>(op.sa(), op.sb(), [&](auto A, auto B) {
 #pragma unroll
             for (int e = 0; e < E; ++e)
                 acc_dot(accr, acci, R.v[decltype(B)::value][e], cmul(((e >> I) & 1) ? d1 : d0, R.v[decltype(A)::value][e]));
@@ -79,7 +81,7 @@ __device__ __forceinline__ void reg_phase_reg(Regs<T, NS, RB> &R, const TileOp &
     }
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
-        if (!((op.smask >> s) & 1u)) continue;
+        if (!((op.smask() >> s) & 1u)) continue;
 #pragma unroll
         for (int e = 0; e < E; ++e) R.v[s][e] = cmul(((e >> I) & 1) ? d1 : d0, R.v[s][e]);
     }
@@ -87,11 +89,11 @@ __device__ __forceinline__ void reg_phase_reg(Regs<T, NS, RB> &R, const TileOp &
 
 // One-bit phase, no controls, on a bit that is fixed per thread.
 template <typename T, int NS, int RB>
-__device__ __forceinline__ void reg_phase_thread(Regs<T, NS, RB> &R, const TileOp &op, typename VecT<T>::type f,
+__device__ __forceinline__ void reg_phase_thread(Regs<T, NS, RB> &R, const OpView &op, typename VecT<T>::type f,
                                                  double &accr, double &acci) {
     constexpr int E = 1 << RB;
-    if (op.flags & TF_DOT) {
-        with_pair<NS>(op.sa, op.sb, [&](auto A, auto B) {
+    if (op.flags() & TF_DOT) {
+        with_pair<NS>(op.sa(), op.sb(), [&](auto A, auto B) {
 #pragma unroll
             for (int e = 0; e < E; ++e)
                 acc_dot(accr, acci, R.v[decltype(B)::value][e], cmul(f, R.v[decltype(A)::value][e]));
@@ -100,22 +102,22 @@ __device__ __forceinline__ void reg_phase_thread(Regs<T, NS, RB> &R, const TileO
     }
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
-        if (!((op.smask >> s) & 1u)) continue;
+        if (!((op.smask() >> s) & 1u)) continue;
 #pragma unroll
         for (int e = 0; e < E; ++e) R.v[s][e] = cmul(f, R.v[s][e]);
     }
 }
 
 template <typename T, int NS, int RB, int I>
-__device__ __forceinline__ void reg_dense1(Regs<T, NS, RB> &R, const TileOp &op, const double2 *coef, uint64_t gbt,
+__device__ __forceinline__ void reg_dense1(Regs<T, NS, RB> &R, const OpView &op, uint64_t gbt,
                                            const uint64_t (&rg)[kMaxRegBits], double &accr, double &acci) {
     using V = typename VecT<T>::type;
     constexpr int E = 1 << RB;
-    const V m00 = ld_coef<T>(coef, op.coef_off + 0), m01 = ld_coef<T>(coef, op.coef_off + 1);
-    const V m10 = ld_coef<T>(coef, op.coef_off + 2), m11 = ld_coef<T>(coef, op.coef_off + 3);
-    const uint64_t gcm = op.gcmask, gcv = op.gcval;
-    if (op.flags & TF_DOT) {
-        with_pair<NS>(op.sa, op.sb, [&](auto A, auto B) {
+    const V m00 = op.template c<T>(0), m01 = op.template c<T>(1);
+    const V m10 = op.template c<T>(2), m11 = op.template c<T>(3);
+    const uint64_t gcm = op.gcmask(), gcv = op.gcval();
+    if (op.flags() & TF_DOT) {
+        with_pair<NS>(op.sa(), op.sb(), [&](auto A, auto B) {
             constexpr int sa = decltype(A)::value, sb = decltype(B)::value;
 #pragma unroll
             for (int e = 0; e < E; ++e) {
@@ -136,7 +138,7 @@ __device__ __forceinline__ void reg_dense1(Regs<T, NS, RB> &R, const TileOp &op,
         if (real) {
 #pragma unroll
             for (int s = 0; s < NS; ++s) {
-                if (!((op.smask >> s) & 1u)) continue;
+                if (!((op.smask() >> s) & 1u)) continue;
 #pragma unroll
                 for (int e = 0; e < E; ++e) {
                     if (e & (1 << I)) continue;
@@ -150,7 +152,7 @@ __device__ __forceinline__ void reg_dense1(Regs<T, NS, RB> &R, const TileOp &op,
         }
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
-            if (!((op.smask >> s) & 1u)) continue;
+            if (!((op.smask() >> s) & 1u)) continue;
 #pragma unroll
             for (int e = 0; e < E; ++e) {
                 if (e & (1 << I)) continue;
@@ -170,7 +172,7 @@ __device__ __forceinline__ void reg_dense1(Regs<T, NS, RB> &R, const TileOp &op,
             const bool ok = (gidx<RB>(gbt, rg, e) & gcm) == gcv;
 #pragma unroll
             for (int s = 0; s < NS; ++s) {
-                if (!((op.smask >> s) & 1u)) continue;
+                if (!((op.smask() >> s) & 1u)) continue;
                 const V a0 = R.v[s][e], a1 = R.v[s][e1];
                 const V n0 = rmul2(m00, a0, m01, a1), n1 = rmul2(m10, a0, m11, a1);
                 R.v[s][e] = ok ? n0 : a0;
@@ -186,7 +188,7 @@ __device__ __forceinline__ void reg_dense1(Regs<T, NS, RB> &R, const TileOp &op,
         const bool ok = (gidx<RB>(gbt, rg, e) & gcm) == gcv;
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
-            if (!((op.smask >> s) & 1u)) continue;
+            if (!((op.smask() >> s) & 1u)) continue;
             const V a0 = R.v[s][e], a1 = R.v[s][e1];
             const V n0 = cmul2(m00, a0, m01, a1), n1 = cmul2(m10, a0, m11, a1);
             R.v[s][e] = ok ? n0 : a0;
@@ -196,15 +198,15 @@ __device__ __forceinline__ void reg_dense1(Regs<T, NS, RB> &R, const TileOp &op,
 }
 
 template <typename T, int NS, int RB, int I0, int I1>
-__device__ __forceinline__ void reg_dense2(Regs<T, NS, RB> &R, const TileOp &op, const double2 *coef, uint64_t gbt,
+__device__ __forceinline__ void reg_dense2(Regs<T, NS, RB> &R, const OpView &op, const double2 *coef, uint64_t gbt,
                                            const uint64_t (&rg)[kMaxRegBits], double &accr, double &acci) {
     using V = typename VecT<T>::type;
     constexpr int E = 1 << RB;
     V m[16];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) m[i] = ld_coef<T>(coef, op.coef_off + i);
-    const uint64_t gcm = op.gcmask, gcv = op.gcval;
-    const bool dot = (op.flags & TF_DOT) != 0;
+    for (int i = 0; i < 16; ++i) m[i] = ld_coef<T>(coef, op.coef_off() + i);
+    const uint64_t gcm = op.gcmask(), gcv = op.gcval();
+    const bool dot = (op.flags() & TF_DOT) != 0;
 #pragma unroll
     for (int e = 0; e < E; ++e) {
         if (e & ((1 << I0) | (1 << I1))) continue;
@@ -214,18 +216,18 @@ __device__ __forceinline__ void reg_dense2(Regs<T, NS, RB> &R, const TileOp &op,
             if (!ok) continue;
             V a[4];
 #pragma unroll
-            for (int c = 0; c < 4; ++c) a[c] = pick(R, op.sa, idx[c]);
+            for (int c = 0; c < 4; ++c) a[c] = pick(R, op.sa(), idx[c]);
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const V o = cmul2(m[4 * r], a[0], m[4 * r + 1], a[1]);
                 const V o2 = cmul2(m[4 * r + 2], a[2], m[4 * r + 3], a[3]);
-                acc_dot(accr, acci, pick(R, op.sb, idx[r]), mk<T>(o.x + o2.x, o.y + o2.y));
+                acc_dot(accr, acci, pick(R, op.sb(), idx[r]), mk<T>(o.x + o2.x, o.y + o2.y));
             }
             continue;
         }
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
-            if (!((op.smask >> s) & 1u)) continue;
+            if (!((op.smask() >> s) & 1u)) continue;
             V a[4], o[4];
 #pragma unroll
             for (int c = 0; c < 4; ++c) a[c] = R.v[s][idx[c]];
@@ -243,15 +245,15 @@ __device__ __forceinline__ void reg_dense2(Regs<T, NS, RB> &R, const TileOp &op,
 
 // Diagonal kinds: DIAG (k <= 2), PARITY, PCPHASE, SIGN, CZSET
 template <typename T, int NS, int RB>
-__device__ __forceinline__ void reg_diag(Regs<T, NS, RB> &R, const TileOp &op, const double2 *coef, uint64_t gbt,
+__device__ __forceinline__ void reg_diag(Regs<T, NS, RB> &R, const OpView &op, const TileOp &tail, const double2 *coef, uint64_t gbt,
                                          const uint64_t (&rg)[kMaxRegBits], double &accr, double &acci) {
     using V = typename VecT<T>::type;
     constexpr int E = 1 << RB;
-    const uint32_t kind = op.kind;
-    const bool dot = (op.flags & TF_DOT) != 0;
-    const uint64_t gcm = op.gcmask, gcv = op.gcval;
+    const uint32_t kind = op.kind();
+    const bool dot = (op.flags() & TF_DOT) != 0;
+    const uint64_t gcm = op.gcmask(), gcv = op.gcval();
     if (kind == TOP_SIGN || kind == TOP_CZSET) {
-        const uint32_t nz = op.nz;
+        const uint32_t nz = op.nz();
 #pragma unroll
         for (int e = 0; e < E; ++e) {
             const uint64_t g = gidx<RB>(gbt, rg, e);
@@ -260,12 +262,12 @@ __device__ __forceinline__ void reg_diag(Regs<T, NS, RB> &R, const TileOp &op, c
                 neg = (g & gcm) == gcv;
             } else {
                 uint32_t p = 0;
-                for (uint32_t i = 0; i < nz; ++i) p += __popcll(g & (g >> op.sd[i]) & op.sm[i]);
+                for (uint32_t i = 0; i < nz; ++i) p += __popcll(g & (g >> tail.sd[i]) & tail.sm[i]);
                 neg = (p & 1u) != 0;
             }
 #pragma unroll
             for (int s = 0; s < NS; ++s) {
-                if (!((op.smask >> s) & 1u)) continue;
+                if (!((op.smask() >> s) & 1u)) continue;
                 R.v[s][e] = neg ? cneg(R.v[s][e]) : R.v[s][e];
             }
         }
@@ -273,12 +275,12 @@ __device__ __forceinline__ void reg_diag(Regs<T, NS, RB> &R, const TileOp &op, c
     }
     if (kind == TOP_TPHASE) {
         // product of one-bit factors on bits fixed per thread
-        V f = ld_coef<T>(coef, op.coef_off + ((gbt >> op.gpos[0]) & 1ull));
-        for (uint32_t j = 1; j < op.k; ++j)
-            f = cmul(ld_coef<T>(coef, op.coef_off + 2 * j + ((gbt >> op.gpos[j]) & 1ull)), f);
+        V f = ld_coef<T>(coef, op.coef_off() + ((gbt >> tail.gpos[0]) & 1ull));
+        for (uint32_t j = 1; j < op.k(); ++j)
+            f = cmul(ld_coef<T>(coef, op.coef_off() + 2 * j + ((gbt >> tail.gpos[j]) & 1ull)), f);
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
-            if (!((op.smask >> s) & 1u)) continue;
+            if (!((op.smask() >> s) & 1u)) continue;
 #pragma unroll
             for (int e = 0; e < E; ++e) R.v[s][e] = cmul(f, R.v[s][e]);
         }
@@ -287,18 +289,18 @@ __device__ __forceinline__ void reg_diag(Regs<T, NS, RB> &R, const TileOp &op, c
     if (kind == TOP_RPHASE) {
 #pragma unroll
         for (int e = 0; e < E; ++e) {
-            const V f = ld_coef<T>(coef, op.coef_off + e);
+            const V f = ld_coef<T>(coef, op.coef_off() + e);
 #pragma unroll
             for (int s = 0; s < NS; ++s) {
-                if (!((op.smask >> s) & 1u)) continue;
+                if (!((op.smask() >> s) & 1u)) continue;
                 R.v[s][e] = cmul(f, R.v[s][e]);
             }
         }
         return;
     }
-    if (kind == TOP_DIAG && op.k == 1 && gcm == 0) {
-        const V d0 = ld_coef<T>(coef, op.coef_off), d1 = ld_coef<T>(coef, op.coef_off + 1);
-        const uint64_t b = 1ull << op.gpos[0];
+    if (kind == TOP_DIAG && op.k() == 1 && gcm == 0) {
+        const V d0 = op.template c<T>(0), d1 = op.template c<T>(1);
+        const uint64_t b = 1ull << op.gp0();
         int r = -1;
 #pragma unroll
         for (int i = 0; i < RB; ++i)
@@ -311,21 +313,22 @@ __device__ __forceinline__ void reg_diag(Regs<T, NS, RB> &R, const TileOp &op, c
         default: reg_phase_thread<T, NS, RB>(R, op, (gbt & b) ? d1 : d0, accr, acci); return;
         }
     }
-    const int k = static_cast<int>(op.k);
+    const int k = static_cast<int>(op.k());
     V d[4];
     const int nd = kind == TOP_DIAG ? (1 << k) : 2;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) d[i] = i < nd ? ld_coef<T>(coef, op.coef_off + i) : d[0];
+    for (int i = 0; i < 4; ++i) d[i] = i < nd ? op.template c<T>(i) : d[0];
 #pragma unroll
     for (int e = 0; e < E; ++e) {
         const uint64_t g = gidx<RB>(gbt, rg, e);
         const bool ok = (g & gcm) == gcv;
         uint32_t idx = 0;
         if (kind == TOP_PARITY) {
-            idx = __popcll(g & op.gpmask) & 1u;
+            idx = __popcll(g & op.gpmask()) & 1u;
         } else {
-            for (int j = 0; j < k; ++j) idx |= static_cast<uint32_t>((g >> op.gpos[j]) & 1ull) << (k - 1 - j);
-            if (kind == TOP_PCPHASE) idx = idx < op.pc_dim ? 0u : 1u;
+            for (int j = 0; j < k; ++j)
+                idx |= static_cast<uint32_t>((g >> (j == 0 ? op.gp0() : j == 1 ? op.gp1() : tail.gpos[j])) & 1ull) << (k - 1 - j);
+            if (kind == TOP_PCPHASE) idx = idx < op.pc_dim() ? 0u : 1u;
         }
         // two-level select on the index bits (a select chain on idx became a
         // dynamically indexed private array, i.e. scratch memory)
@@ -333,12 +336,12 @@ __device__ __forceinline__ void reg_diag(Regs<T, NS, RB> &R, const TileOp &op, c
         const V f23 = (idx & 1u) ? d[3] : d[2];
         const V f = (idx & 2u) ? f23 : f01;
         if (dot) {
-            if (ok) acc_dot(accr, acci, pick(R, op.sb, e), cmul(f, pick(R, op.sa, e)));
+            if (ok) acc_dot(accr, acci, pick(R, op.sb(), e), cmul(f, pick(R, op.sa(), e)));
             continue;
         }
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
-            if (!((op.smask >> s) & 1u)) continue;
+            if (!((op.smask() >> s) & 1u)) continue;
             const V x = R.v[s][e];
             R.v[s][e] = ok ? cmul(f, x) : x;
         }
@@ -346,15 +349,15 @@ __device__ __forceinline__ void reg_diag(Regs<T, NS, RB> &R, const TileOp &op, c
 }
 
 template <typename T, int NS, int RB, bool WIDE>
-__device__ __forceinline__ void reg_apply(Regs<T, NS, RB> &R, const TileOp &op, const double2 *coef, uint64_t gbt,
+__device__ __forceinline__ void reg_apply(Regs<T, NS, RB> &R, const OpView &op, const TileOp &tail, const double2 *coef, uint64_t gbt,
                                           const uint64_t (&rg)[kMaxRegBits], double &accr, double &acci) {
-    const uint32_t kind = op.kind;
+    const uint32_t kind = op.kind();
     if (kind == TOP_DENSE1) {
-        switch (op.lpos[0]) {
-        case 0: reg_dense1<T, NS, RB, 0>(R, op, coef, gbt, rg, accr, acci); break;
-        case 1: if constexpr (RB > 1) reg_dense1<T, NS, RB, 1>(R, op, coef, gbt, rg, accr, acci); break;
-        case 2: if constexpr (RB > 2) reg_dense1<T, NS, RB, 2>(R, op, coef, gbt, rg, accr, acci); break;
-        case 3: if constexpr (RB > 3) reg_dense1<T, NS, RB, 3>(R, op, coef, gbt, rg, accr, acci); break;
+        switch (op.lp0()) {
+        case 0: reg_dense1<T, NS, RB, 0>(R, op, gbt, rg, accr, acci); break;
+        case 1: if constexpr (RB > 1) reg_dense1<T, NS, RB, 1>(R, op, gbt, rg, accr, acci); break;
+        case 2: if constexpr (RB > 2) reg_dense1<T, NS, RB, 2>(R, op, gbt, rg, accr, acci); break;
+        case 3: if constexpr (RB > 3) reg_dense1<T, NS, RB, 3>(R, op, gbt, rg, accr, acci); break;
         default: break;
         }
     } else if (kind == TOP_DENSE2) {
@@ -363,7 +366,7 @@ __device__ __forceinline__ void reg_apply(Regs<T, NS, RB> &R, const TileOp &op, 
     case (a)*4 + (b):                                                                                        \
         if constexpr ((a) < RB && (b) < RB) reg_dense2<T, NS, RB, a, b>(R, op, coef, gbt, rg, accr, acci);   \
         break;
-        switch (op.lpos[0] * 4 + op.lpos[1]) {
+        switch (op.lp0() * 4 + op.lp1()) {
             LQ_D2(0, 1) LQ_D2(0, 2) LQ_D2(0, 3) LQ_D2(1, 0) LQ_D2(1, 2) LQ_D2(1, 3)
             LQ_D2(2, 0) LQ_D2(2, 1) LQ_D2(2, 3) LQ_D2(3, 0) LQ_D2(3, 1) LQ_D2(3, 2)
         default: break;
@@ -371,7 +374,7 @@ __device__ __forceinline__ void reg_apply(Regs<T, NS, RB> &R, const TileOp &op, 
 #undef LQ_D2
         }
     } else {
-        reg_diag<T, NS, RB>(R, op, coef, gbt, rg, accr, acci);
+        reg_diag<T, NS, RB>(R, op, tail, coef, gbt, rg, accr, acci);
     }
 }
 
@@ -384,6 +387,7 @@ __device__ __forceinline__ void reg_apply(Regs<T, NS, RB> &R, const TileOp &op, 
 template <typename T, int NS, int RB, bool WIDE>
 __global__ __launch_bounds__(kBlock) void tile_reg_kernel(TileRegArgs a, typename VecT<T>::type *__restrict__ sv0,
                                                          typename VecT<T>::type *__restrict__ sv1,
+                                                         const OpHead *__restrict__ heads,
                                                          const TileOp *__restrict__ ops,
                                                          const TileStage *__restrict__ stages,
                                                          const double2 *__restrict__ coef,
@@ -399,16 +403,14 @@ __global__ __launch_bounds__(kBlock) void tile_reg_kernel(TileRegArgs a, typenam
     const uint64_t tile = static_cast<uint64_t>(blockIdx.x) + static_cast<uint64_t>(blockIdx.y) * gridDim.x;
     if (tile >= a.ntiles) return; // uniform over the block
     const int kt = a.g.kt;        // == 8 + RB
-    const int c = a.g.c;
     const uint32_t tsize = 1u << kt;
 
-    uint64_t base = 0;
-    for (int j = 0; j < a.g.nout; ++j) base |= ((tile >> j) & 1ull) << a.g.ob[j];
-    auto spread = [&](uint32_t l) -> uint64_t {
-        uint64_t s = l & ((1u << c) - 1u);
-        for (int b = c; b < kt; ++b) s |= static_cast<uint64_t>((l >> b) & 1u) << a.g.tb[b];
-        return s;
-    };
+    const uint64_t base = deposit_bits(tile, a.g.ob, a.g.nout);
+    auto spread = [&](uint32_t l) -> uint64_t { return spread_bits(l, a.g.tb); };
+    if (a.ntiles <= kWarmTiles) {
+        warm_program(heads, a.nops * static_cast<uint32_t>(sizeof(OpHead)));
+        warm_program(stages, a.nstages * static_cast<uint32_t>(sizeof(TileStage)));
+    }
     if (a.nslots) {
         for (uint32_t i = tid; i < (kBlock / 64) * kMaxPassDots; i += kBlock)
             dred[i / kMaxPassDots][i % kMaxPassDots] = make_double2(0.0, 0.0);
@@ -468,6 +470,13 @@ __global__ __launch_bounds__(kBlock) void tile_reg_kernel(TileRegArgs a, typenam
     };
 
     bool in_lds = false;
+    OpView next = OpView::load(heads);
+    // op oi, with the next one's head put in flight while it runs
+    auto fetch = [&](uint32_t oi) {
+        const OpView op = next;
+        next = OpView::load(heads + (oi + 1 < a.nops ? oi + 1 : oi));
+        return op;
+    };
     for (uint32_t si = 0; si < a.nstages; ++si) {
         const TileStage &st = stages[si];
         if (st.kind == STAGE_REG) {
@@ -487,12 +496,12 @@ __global__ __launch_bounds__(kBlock) void tile_reg_kernel(TileRegArgs a, typenam
 #pragma unroll
             for (int i = 0; i < kMaxRegBits; ++i) rg[i] = i < RB ? (1ull << a.g.tb[cr[i]]) : 0ull;
             for (uint32_t oi = st.op_begin; oi < st.op_end; ++oi) {
-                const TileOp &op = ops[oi];
+                const OpView op = fetch(oi);
                 double accr = 0.0, acci = 0.0;
-                reg_apply<T, NS, RB, WIDE>(R, op, coef, gbt, rg, accr, acci);
-                if (op.flags & TF_DOT) {
+                reg_apply<T, NS, RB, WIDE>(R, op, ops[oi], coef, gbt, rg, accr, acci);
+                if (op.flags() & TF_DOT) {
                     wave_sum(accr, acci);
-                    if ((tid & 63u) == 0) dred[tid >> 6][op.slot] = make_double2(accr, acci);
+                    if ((tid & 63u) == 0) dred[tid >> 6][op.slot()] = make_double2(accr, acci);
                 }
             }
         } else if constexpr (WIDE) {
@@ -503,18 +512,18 @@ __global__ __launch_bounds__(kBlock) void tile_reg_kernel(TileRegArgs a, typenam
                 in_lds = true;
             }
             for (uint32_t oi = st.op_begin; oi < st.op_end; ++oi) {
-                const TileOp &op = ops[oi];
-                if ((base & op.ocmask) == op.ocval) {
+                const OpView op = fetch(oi);
+                if ((base & op.ocmask()) == op.ocval()) {
                     double accr = 0.0, acci = 0.0;
-                    lds_apply_op<T, NS, true>(op, lds, tsize, base, coef, accr, acci);
-                    if (op.flags & TF_DOT) {
+                    lds_apply_op<T, NS, true>(op, ops[oi], lds, tsize, base, coef, accr, acci);
+                    if (op.flags() & TF_DOT) {
                         wave_sum(accr, acci);
-                        if ((tid & 63u) == 0) dred[tid >> 6][op.slot] = make_double2(accr, acci);
+                        if ((tid & 63u) == 0) dred[tid >> 6][op.slot()] = make_double2(accr, acci);
                     }
-                } else if (op.flags & TF_ZERO_UNCTRL) {
+                } else if (op.flags() & TF_ZERO_UNCTRL) {
 #pragma unroll
                     for (int s = 0; s < NS; ++s)
-                        if ((op.smask >> s) & 1u)
+                        if ((op.smask() >> s) & 1u)
                             for (uint32_t l = tid; l < tsize; l += kBlock) lds[s * tsize + l] = mk<T>(T(0), T(0));
                 }
                 __syncthreads();
@@ -572,10 +581,10 @@ template <typename T> void launch_tile_reg(const TileRegArgs &a, size_t lds_byte
     do {                                                                                                       \
         if (a.wide)                                                                                            \
             hipLaunchKernelGGL((tile_reg_kernel<T, NS_, RB_, true>), grid, dim3(kBlock), lds_bytes, s, a, p0,  \
-                               p1, a.ops, a.stages, a.coef, a.partials);                                       \
+                               p1, a.heads, a.ops, a.stages, a.coef, a.partials);                                       \
         else                                                                                                   \
             hipLaunchKernelGGL((tile_reg_kernel<T, NS_, RB_, false>), grid, dim3(kBlock), lds_bytes, s, a, p0, \
-                               p1, a.ops, a.stages, a.coef, a.partials);                                       \
+                               p1, a.heads, a.ops, a.stages, a.coef, a.partials);                                       \
     } while (0)
     if (a.ns == 1) {
         switch (rb) {

@@ -100,6 +100,21 @@ struct alignas(16) TileOp {
     int32_t gpos[kMaxTileOpTargets]; // global bit of target j (target 0 = local MSB)
 };
 
+// What the interpreting kernels read of an op, in three 64-byte lines: its
+// scalar fields, its first two targets and its first four coefficients. A wave
+// reads a whole head with one load of one word per lane (OpView), the next
+// op's while one runs; only ops with more targets, terms or coefficients go to
+// the TileOp and the coefficient buffer.
+struct alignas(64) OpHead {
+    uint32_t kind, flags, k, smask;
+    uint32_t sa, sb, slot, nz;
+    uint32_t lcmask, lcval, lxmask, lzmask;
+    int32_t lp0, lp1, gp0, gp1; // lpos / gpos of targets 0 and 1
+    uint64_t ocmask, ocval, omask, gcmask;
+    uint64_t gcval, gpmask, coef_off, pc_dim;
+    double c[8];                // coefficients 0..3, (re, im)
+};
+
 struct TileGeom {
     int32_t n;                // qubits
     int32_t kt;               // tile bits
