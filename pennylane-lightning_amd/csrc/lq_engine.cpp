@@ -710,6 +710,76 @@ std::vector<PassPlan> plan_search(const std::vector<LOp> &prog, const PlanConfig
     return passes;
 }
 
+// Complete plans at rest, by structure and precision: a plan whose kernels are
+// all compiled is lent to one program at a time, which refills its
+// coefficients; a second program of the same structure meanwhile takes the
+// ordinary way through the plan cache and the kernel lookups. At most
+// kMaxPerHome wait per structure and kMaxResting in all.
+struct PlanHome {
+    std::vector<StateVector::Planned> resting;
+    bool dropped = false; // no longer in the table: keeps nothing (under the pool's mutex)
+    std::atomic<int> single_passes{0}; // of the one-observable sweep a group's plan competes with
+};
+
+namespace {
+struct PlanPool {
+    std::mutex mu;
+    std::unordered_map<std::string, std::shared_ptr<PlanHome>> map;
+    std::deque<std::string> order;
+    size_t resting = 0;
+    static constexpr size_t kMaxHomes = 256, kMaxPerHome = 2, kMaxResting = 256;
+    static PlanPool &get() {
+        static PlanPool *p = new PlanPool(); // plans may come back from static destructors
+        return *p;
+    }
+    std::shared_ptr<PlanHome> home(const std::string &key, StateVector::Planned *lent) {
+        std::vector<std::shared_ptr<PlanHome>> dropped; // freed outside the lock
+        std::lock_guard<std::mutex> lk(mu);
+        auto it = map.find(key);
+        if (it == map.end()) {
+            it = map.emplace(key, std::make_shared<PlanHome>()).first;
+            order.push_back(key);
+            if (order.size() > kMaxHomes) {
+                auto old = map.find(order.front());
+                resting -= old->second->resting.size();
+                old->second->dropped = true;
+                dropped.push_back(old->second);
+                map.erase(old);
+                order.pop_front();
+                it = map.find(key);
+            }
+        }
+        PlanHome &h = *it->second;
+        if (!h.resting.empty()) {
+            *lent = std::move(h.resting.back());
+            h.resting.pop_back();
+            --resting;
+        }
+        return it->second;
+    }
+};
+} // namespace
+
+void StateVector::Planned::give_back() {
+    if (!home) return;
+    std::shared_ptr<PlanHome> h = std::move(home);
+    home.reset();
+    if (passes.empty()) return;
+    for (size_t p = 0; p < passes.size(); ++p)
+        if (!fns[p] && !passes[p].dense) return;
+    PlanPool &pool = PlanPool::get();
+    std::lock_guard<std::mutex> lk(pool.mu);
+    if (h->dropped || h->resting.size() >= PlanPool::kMaxPerHome || pool.resting >= PlanPool::kMaxResting) return;
+    StateVector::Planned p;
+    p.passes = std::move(passes);
+    p.fns = std::move(fns);
+    p.geo = std::move(geo);
+    p.ns = ns;
+    p.device = device;
+    h->resting.push_back(std::move(p));
+    ++pool.resting;
+}
+
 StateVector::Planned StateVector::plan(const std::vector<LOp> &prog, int ns, bool forms) {
     LQ_ABORT_IF(ns < 1 || ns > kMaxStates, "too many states in one program");
     Planned out;
@@ -723,8 +793,10 @@ StateVector::Planned StateVector::plan(const std::vector<LOp> &prog, int ns, boo
     cfg.low_bits = t.low_bits >= 0 ? t.low_bits : (dtype_ ? 4 : 5);
     cfg.budget = t.budget > 0 ? t.budget : 24.0;
     cfg.dense_passes = true;
-    // a state that is one tile gains nothing from a second pass
-    if (t.budget <= 0 && n_ <= cfg.kt_max) cfg.budget = 1e9;
+    cfg.keep_grouping = dtype_ == 0;
+    // a state that is one tile gains nothing from a second pass (complex64
+    // keeps its passes with its grouping)
+    if (t.budget <= 0 && n_ <= cfg.kt_max && dtype_) cfg.budget = 1e9;
     // register-resident passes for tiles of 11 or 12 bits with one or two states
     const int ktr = std::min(cfg.kt_max, 8 + kMaxRegBits);
     if (t.reg && ns <= 2 && n_ >= 11 && ktr >= 11) {
@@ -788,7 +860,22 @@ StateVector::Planned StateVector::plan(const std::vector<LOp> &prog, int ns, boo
             scfg.max_dots = std::min(kMaxJitPassDots, kMaxPassDots * (ns - 1));
         }
         std::vector<LOp> split = prog;
-        split_1q_rotations(split);
+        split_1q_rotations(split, dtype_ == 0);
+        if (t.plan_cache) {
+            std::string key = plan_structure_key(split, scfg);
+            key.push_back(static_cast<char>('0' + dtype_ + (t.plan_search.load() ? 2 : 0)));
+            int dev = -1;
+            (void)hipGetDevice(&dev);
+            std::shared_ptr<PlanHome> home = PlanPool::get().home(key, &out);
+            if (!out.passes.empty() && out.device == dev && refresh_plan_coefs(out.passes, split)) {
+                out.home = std::move(home);
+                return out;
+            }
+            out = Planned{};
+            out.ns = ns;
+            out.device = dev;
+            out.home = std::move(home);
+        }
         passes = (t.budget <= 0 && t.plan_search.load() && n_ >= kPlanSearchQubits) ? plan_search(split, scfg)
                                                                               : plan_cached(split, scfg);
         const size_t missing = lookup_all(fns);
@@ -808,6 +895,7 @@ StateVector::Planned StateVector::plan(const std::vector<LOp> &prog, int ns, boo
                 passes.swap(plain);
                 fns.assign(passes.size(), nullptr);
                 geo.assign(passes.size(), nullptr);
+                out.home.reset(); // not the plan of that structure
             }
         }
     } else {
@@ -2062,24 +2150,33 @@ void adjoint_jacobian(StateVector &sv, const OpsList &ops, const std::vector<std
         w.planned = sv.plan(prog, 1 + static_cast<int>(m));
         return w;
     };
-    Sweep single = make_sweep(1);
-    Sweep group;
+    Sweep single, group;
     const int grouping = tuning().adjoint_group.load();
     if (nobs > 1 && grouping > 0) {
         group = make_sweep(std::min<size_t>(3, nobs));
+        // the single sweep is built when it runs (observables left over) or
+        // its pass count is not known yet
+        PlanHome *home = group.planned.home.get();
+        int s_passes = home ? home->single_passes.load() : 0;
+        if (s_passes == 0 || nobs % group.m != 0) {
+            single = make_sweep(1);
+            s_passes = static_cast<int>(single.planned.passes.size());
+            if (home && single.planned.all_specialised()) home->single_passes.store(s_passes);
+        }
         // state traffic of the sweeps (passes x states each pass streams):
         // a group against one sweep per observable
         const double g_cost = static_cast<double>(group.planned.passes.size()) * static_cast<double>(1 + group.m);
-        const double s_cost = static_cast<double>(single.planned.passes.size()) * 2.0 * static_cast<double>(group.m);
+        const double s_cost = static_cast<double>(s_passes) * 2.0 * static_cast<double>(group.m);
         const bool ready = group.planned.all_specialised();
         const bool take = ready && (grouping == 2 || g_cost < s_cost);
         if (tuning().adjoint_debug)
             std::fprintf(stderr, "[lq adjoint] observables %zu: group of %zu in %zu passes (specialised %d), single %zu "
                                  "passes: %s\n",
-                         nobs, group.m, group.planned.passes.size(), ready ? 1 : 0, single.planned.passes.size(),
+                         nobs, group.m, group.planned.passes.size(), ready ? 1 : 0, static_cast<size_t>(s_passes),
                          take ? "groups" : "one per sweep");
         if (!take) group = Sweep{};
     }
+    if (single.m == 0 && (group.m == 0 || nobs % group.m != 0)) single = make_sweep(1);
     std::vector<double> out(nobs * ntp, 0.0);
     for (size_t o0 = 0; o0 < nobs;) {
         const Sweep &w = (group.m > 0 && nobs - o0 >= group.m) ? group : single;

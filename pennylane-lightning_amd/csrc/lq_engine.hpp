@@ -149,6 +149,8 @@ struct EngineTuning {
 };
 EngineTuning &tuning();
 
+struct PlanHome;
+
 class StateVector {
   public:
     StateVector(int n, int dtype);
@@ -238,6 +240,26 @@ class StateVector {
         std::vector<hipFunction_t> fns; // specialised kernel per pass, or null
         std::vector<const std::vector<uint64_t> *> geo; // its bit-position table (null or empty: none)
         int ns = 0;
+        int device = -1;                // whose kernels fns are
+        // where a plan with all its kernels goes back to when it is done with
+        // (a program of the same structure then only refills its coefficients)
+        std::shared_ptr<PlanHome> home;
+        Planned() = default;
+        Planned(Planned &&) = default;
+        Planned &operator=(Planned &&o) noexcept {
+            if (this != &o) {
+                give_back();
+                passes = std::move(o.passes);
+                fns = std::move(o.fns);
+                geo = std::move(o.geo);
+                ns = o.ns;
+                device = o.device;
+                home = std::move(o.home);
+            }
+            return *this;
+        }
+        ~Planned() { give_back(); }
+        void give_back();
         bool all_specialised() const {
             for (hipFunction_t f : fns)
                 if (!f) return false;

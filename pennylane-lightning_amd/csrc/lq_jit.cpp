@@ -878,13 +878,17 @@ class Gen {
         const std::string accf = pred ? "accp(" : "acc(";
         const std::string gsuf = pred ? ", gd)" : ")";
         const uint64_t off = t.coef_off;
-        if (dot && (t.flags & (TF_DOT_X | TF_DOT_Y | TF_DOT_Z))) {
+        // class dots and exchanges in complex128 only: in single precision the
+        // compiler contracts the other gates' products otherwise beside these
+        // forms, which moves the amplitudes' last bits (see
+        // PlanConfig::keep_grouping)
+        if (dot && dtype_ && (t.flags & (TF_DOT_X | TF_DOT_Y | TF_DOT_Z))) {
             emit_class_dot(t, A, B, pred);
             emit_flush(t);
             o << "  }\n";
             return;
         }
-        if ((t.flags & TF_SWAP) && !dot) {
+        if ((t.flags & TF_SWAP) && !dot && dtype_) {
             // X or SWAP: amplitudes change places, in the registers' names
             // alone unless a control is a thread bit
             for (int e = 0; e < E_; ++e) {

@@ -207,8 +207,78 @@ void controls_to_mask(int n, const uint32_t *ctrls, const uint8_t *cvals, int nc
 }
 } // namespace
 
+namespace {
+// Lowered forms of the gates without parameters and of the generators, made
+// once on bits 0..nw-1 (wires[j] on bit nw-1-j): lowering one of them is then a
+// copy with its bits put in place.
+struct Template {
+    bool known = false;
+    LOp op;
+    double scale = 0.0;
+};
+constexpr int kGates = static_cast<int>(GateId::Count);
+
+LOp place_template(const LOp &t, const int *tb, int nw, uint64_t cm, uint64_t cv) {
+    LOp op = t;
+    for (int j = 0; j < op.k; ++j) op.bits[j] = tb[nw - 1 - t.bits[j]];
+    op.cmask = cm;
+    op.cval = cv;
+    for (int j = 0; j < nw; ++j) {
+        const uint64_t from = 1ull << (nw - 1 - j), to = 1ull << tb[j];
+        if (t.cmask & from) op.cmask |= to;
+        if (t.cval & from) op.cval |= to;
+    }
+    return op;
+}
+
+const Template &gate_template(GateId g, bool inverse) {
+    static const std::vector<Template> table = [] {
+        std::vector<Template> t(2 * kGates);
+        for (int i = 0; i < kGates; ++i) {
+            const GateInfo &info = gate_info(static_cast<GateId>(i));
+            if (info.nparams != 0 || info.nwires < 1 || info.nwires > 4 || static_cast<GateId>(i) == GateId::Identity)
+                continue;
+            std::vector<int> tb;
+            for (int j = 0; j < info.nwires; ++j) tb.push_back(info.nwires - 1 - j);
+            for (int inv = 0; inv < 2; ++inv) {
+                Template &x = t[2 * i + inv];
+                x.op = lower_matrix(gate_matrix(static_cast<GateId>(i), nullptr, inv != 0, info.nwires), tb, 0, 0, false);
+                x.known = true;
+            }
+        }
+        return t;
+    }();
+    return table[2 * static_cast<size_t>(g) + (inverse ? 1 : 0)];
+}
+
+const Template &generator_template(GateId g) {
+    static const std::vector<Template> table = [] {
+        std::vector<Template> t(kGates);
+        for (int i = 0; i < kGates; ++i) {
+            const GateInfo &info = gate_info(static_cast<GateId>(i));
+            if (!info.has_generator || info.nwires < 1 || info.nwires > 4) continue;
+            std::vector<int> tb;
+            for (int j = 0; j < info.nwires; ++j) tb.push_back(info.nwires - 1 - j);
+            Generator gen = gate_generator(static_cast<GateId>(i), info.nwires);
+            t[i].op = lower_matrix(gen.g, tb, 0, 0, true);
+            t[i].scale = gen.scale;
+            t[i].known = true;
+        }
+        return t;
+    }();
+    return table[static_cast<size_t>(g)];
+}
+} // namespace
+
 LOp lower_gate(int n, GateId g, const uint32_t *wires, int nw, const uint32_t *ctrls, const uint8_t *cvals, int nc,
                bool inverse, const double *params) {
+    if (const Template &t = gate_template(g, inverse); t.known && nw == gate_info(g).nwires) {
+        uint64_t cm, cv;
+        controls_to_mask(n, ctrls, cvals, nc, &cm, &cv);
+        int tb[4];
+        for (int j = 0; j < nw; ++j) tb[j] = phys_bit(n, wires[j]);
+        return place_template(t.op, tb, nw, cm, cv);
+    }
     uint64_t cm, cv;
     controls_to_mask(n, ctrls, cvals, nc, &cm, &cv);
     std::vector<int> tb(nw);
@@ -249,13 +319,44 @@ LOp lower_gate(int n, GateId g, const uint32_t *wires, int nw, const uint32_t *c
         op.coef = {std::exp(cd(0.0, inverse ? params[0] : -params[0]))};
         return op;
     }
-    return lower_matrix(gate_matrix(g, params, inverse, nw), tb, cm, cv, false);
+    std::vector<cd> m = gate_matrix(g, params, inverse, nw);
+    if (nw == 1 && m.size() == 4 && m[1] != cd(0.0) && m[2] != cd(0.0)) {
+        // nothing for lower_matrix to take apart
+        LOp op;
+        op.kind = TOP_DENSE1;
+        op.k = 1;
+        op.bits[0] = tb[0];
+        op.cmask = cm;
+        op.cval = cv;
+        op.coef = std::move(m);
+        return op;
+    }
+    if (nw == 1 && m.size() == 4 && m[1] == cd(0.0) && m[2] == cd(0.0) && m[0] != m[3] && m[0] != cd(1.0) &&
+        m[3] != cd(1.0)) {
+        LOp op; // RZ
+        op.kind = TOP_DIAG;
+        op.k = 1;
+        op.bits[0] = tb[0];
+        op.cmask = cm;
+        op.cval = cv;
+        op.coef = {m[0], m[3]};
+        return op;
+    }
+    return lower_matrix(std::move(m), tb, cm, cv, false);
 }
 
 LOp lower_generator(int n, GateId g, const uint32_t *wires, int nw, const uint32_t *ctrls, const uint8_t *cvals,
                     int nc, double *scale) {
     uint64_t cm, cv;
     controls_to_mask(n, ctrls, cvals, nc, &cm, &cv);
+    if (const Template &t = generator_template(g); t.known && nw == gate_info(g).nwires) {
+        int tb4[4];
+        for (int j = 0; j < nw; ++j) tb4[j] = phys_bit(n, wires[j]);
+        LOp op = place_template(t.op, tb4, nw, cm, cv);
+        op.flags |= TF_ZERO_UNCTRL;
+        *scale = t.scale;
+        return op;
+    }
     std::vector<int> tb(nw);
     for (int j = 0; j < nw; ++j) tb[j] = phys_bit(n, wires[j]);
     LOp op;
@@ -329,26 +430,55 @@ size_t absorb_into_product(std::vector<LOp> &prog, std::vector<cd> &f) {
     return folded;
 }
 
-void split_1q_rotations(std::vector<LOp> &prog) {
+void split_1q_rotations(std::vector<LOp> &prog, bool keep_grouping) {
     std::vector<LOp> out;
     out.reserve(prog.size() * 3);
     for (auto &o : prog) {
         const bool candidate = (o.kind == TOP_DENSE1 || o.kind == TOP_DENSEK) && o.k == 1 && o.cmask == 0 &&
-                               !o.is_dot() && !(o.flags & TF_ZERO_UNCTRL) && o.coef.size() == 4 && !o.is_swap();
+                               !o.is_dot() && !(o.flags & TF_ZERO_UNCTRL) && o.coef.size() == 4 &&
+                               (keep_grouping || !o.is_swap());
         if (!candidate) {
             out.push_back(std::move(o));
             continue;
         }
         const cd u00 = o.coef[0], u01 = o.coef[1], u10 = o.coef[2], u11 = o.coef[3];
-        const double gamma = std::arg(u00 * u11 - u01 * u10) / 2.0;
-        const cd eg = std::polar(1.0, -gamma);
-        const cd a = eg * u00, b = eg * u10;
-        const double c = std::abs(a), sn = std::abs(b);
-        const double pa = c > 1e-300 ? std::arg(a) : 0.0, pb = sn > 1e-300 ? std::arg(b) : 0.0;
-        const double alpha = pb - pa, delta = -pa - pb;
-        const cd d1_0 = std::polar(1.0, -delta / 2), d1_1 = std::polar(1.0, delta / 2);
-        const cd d2_0 = std::polar(1.0, gamma - alpha / 2), d2_1 = std::polar(1.0, gamma + alpha / 2);
-        // U' = D2 R D1 with R = [[c, -s], [s, c]]
+        // U = D2 R D1 with R = [[c, -s], [s, c]] from the entries of U, without
+        // angles; D1 = diag(1, .) unless an entry vanishes. The signs go to c
+        // and s (phases from one half of the plane), so that which phases are
+        // exactly 1 or -1 depends on the kind of gate, not on its angles.
+        double c = std::abs(u00), sn = std::abs(u10);
+        cd d1_0(1.0), d1_1, d2_0, d2_1;
+        // rounding next to 1, -1, i, -i does not count
+        auto snap = [](cd ph) {
+            if (std::fabs(ph.imag()) <= 1e-15) return cd(ph.real() < 0.0 ? -1.0 : 1.0, 0.0);
+            if (std::fabs(ph.real()) <= 1e-15) return cd(0.0, ph.imag() < 0.0 ? -1.0 : 1.0);
+            return ph;
+        };
+        auto phase_of = [&](const cd &u, double &m) {
+            cd ph = snap(u / m);
+            if (ph.real() < 0.0 || (ph.real() == 0.0 && ph.imag() < 0.0)) {
+                ph = -ph;
+                m = -m;
+            }
+            return ph;
+        };
+        if (!keep_grouping && c > 1e-100 && sn > 1e-100 && std::abs(u11) > 1e-100) {
+            d2_0 = phase_of(u00, c);
+            d2_1 = phase_of(u10, sn);
+            d1_1 = snap(u11 / std::abs(u11) * std::conj(d2_1) * (c < 0.0 ? -1.0 : 1.0));
+        } else {
+            const double gamma = std::arg(u00 * u11 - u01 * u10) / 2.0;
+            const cd eg = std::polar(1.0, -gamma);
+            const cd a = eg * u00, b = eg * u10;
+            c = std::abs(a);
+            sn = std::abs(b);
+            const double pa = c > 1e-300 ? std::arg(a) : 0.0, pb = sn > 1e-300 ? std::arg(b) : 0.0;
+            const double alpha = pb - pa, delta = -pa - pb;
+            d1_0 = std::polar(1.0, -delta / 2);
+            d1_1 = std::polar(1.0, delta / 2);
+            d2_0 = std::polar(1.0, gamma - alpha / 2);
+            d2_1 = std::polar(1.0, gamma + alpha / 2);
+        }
         const cd r00 = d2_0 * c * d1_0, r01 = d2_0 * (-sn) * d1_1, r10 = d2_1 * sn * d1_0, r11 = d2_1 * c * d1_1;
         const double err = std::max(std::max(std::abs(r00 - u00), std::abs(r01 - u01)),
                                     std::max(std::abs(r10 - u10), std::abs(r11 - u11)));
@@ -368,9 +498,10 @@ void split_1q_rotations(std::vector<LOp> &prog) {
         rot.coef = {cd(c), cd(-sn), cd(sn), cd(c)};
         LOp p2 = p1;
         p2.coef = {d2_0, d2_1};
-        out.push_back(std::move(p1));
+        const cd one(1.0);
+        if (keep_grouping || d1_0 != one || d1_1 != one) out.push_back(std::move(p1)); // RY has none
         out.push_back(std::move(rot));
-        out.push_back(std::move(p2));
+        if (keep_grouping || d2_0 != one || d2_1 != one) out.push_back(std::move(p2));
     }
     // Move each one-bit phase later past the ops it commutes with (anything
     // acting diagonally on its bit or on other states) and fold it into the
@@ -382,29 +513,53 @@ void split_1q_rotations(std::vector<LOp> &prog) {
     auto unit_phase = [](const LOp &o) {
         return std::fabs(std::norm(o.coef[0]) - 1.0) <= 1e-12 && std::fabs(std::norm(o.coef[1]) - 1.0) <= 1e-12;
     };
+    // Walking backwards, a phase only has to look at the next op on its bit
+    // that acts non-diagonally there or is a phase, and at what acts on other
+    // states: per bit, the next op that a phase on it can meet.
     std::vector<char> gone(out.size(), 0);
-    for (size_t i = 0; i < out.size(); ++i) {
-        if (!is_phase(out[i])) continue;
-        const uint64_t bit = 1ull << out[i].bits[0];
-        const size_t lim = std::min(out.size(), i + 4096);
-        for (size_t j = i + 1; j < lim; ++j) {
-            const LOp &o = out[j];
-            if (gone[j]) continue;
-            if (o.is_dot()) {
-                // <b|D^dagger G D|a> = <b|G|a> for a phase on both states and a bit that G acts on diagonally or not at all
-                const uint32_t ab = (1u << o.sa) | (1u << o.sb);
-                if ((out[i].smask & ab) != ab || (o.nmask() & bit) || !unit_phase(out[i])) break;
+    constexpr size_t kNone = static_cast<size_t>(-1);
+    size_t next_on[64];
+    size_t next_any = kNone; // next op or dot that stops phases of the common state set on every bit
+    std::fill(next_on, next_on + 64, kNone);
+    uint32_t common = 0;     // the states of the phases tracked
+    std::vector<size_t> link(out.size(), kNone); // the op that phase i meets first
+    for (size_t i = out.size(); i-- > 0;) {
+        const LOp &o = out[i];
+        if (is_phase(o)) {
+            if (o.smask != common) {
+                // phases on other states: nothing is known about the ops after it
+                std::fill(next_on, next_on + 64, kNone);
+                next_any = i + 1 < out.size() ? i + 1 : kNone;
+                common = o.smask;
+            }
+            link[i] = std::min(next_on[o.bits[0]], next_any);
+            next_on[o.bits[0]] = i;
+            continue;
+        }
+        if (o.is_dot()) {
+            const uint32_t ab = (1u << o.sa) | (1u << o.sb);
+            if ((common & ab) != ab || keep_grouping) {
+                if (common) next_any = i;
                 continue;
             }
-            if (!(o.smask & out[i].smask)) continue;
-            if (is_phase(o) && o.bits[0] == out[i].bits[0] && o.smask == out[i].smask) {
-                out[j].coef[0] *= out[i].coef[0];
-                out[j].coef[1] *= out[i].coef[1];
-                gone[i] = 1;
-                break;
-            }
-            if ((o.nmask() & bit) || o.smask != out[i].smask) break;
+        } else if (o.smask != common) {
+            if (common & o.smask) next_any = i;
+            continue;
         }
+        for (uint64_t m = o.nmask(); m; m &= m - 1) next_on[__builtin_ctzll(m)] = i;
+    }
+    for (size_t i = 0; i < out.size(); ++i) {
+        if (!is_phase(out[i])) continue;
+        size_t j = link[i];
+        if (j == kNone || !is_phase(out[j]) || out[j].bits[0] != out[i].bits[0] || out[j].smask != out[i].smask) continue;
+        if (keep_grouping && j - i >= 4096) continue;
+        // past a dot only when unitary
+        if (!unit_phase(out[i]) && std::any_of(out.begin() + static_cast<long>(i), out.begin() + static_cast<long>(j),
+                                               [](const LOp &o) { return o.is_dot(); }))
+            continue;
+        out[j].coef[0] *= out[i].coef[0];
+        out[j].coef[1] *= out[i].coef[1];
+        gone[i] = 1;
     }
     prog.clear();
     for (size_t i = 0; i < out.size(); ++i)
@@ -1121,7 +1276,7 @@ std::vector<PassPlan> plan_passes(const std::vector<LOp> &ops, const PlanConfig 
         // specialised passes swap the amplitudes of an X or SWAP: a select per
         // word where a control is a thread bit, nothing otherwise
         cost_of[j] = ops[j].cost();
-        if (cfg.lookahead && !ops[j].is_dot() && ops[j].is_swap()) cost_of[j] *= kSwapCost / (ops[j].k == 1 ? 1.0 : 2.5);
+        if (cfg.lookahead && !cfg.keep_grouping && !ops[j].is_dot() && ops[j].is_swap()) cost_of[j] *= kSwapCost / (ops[j].k == 1 ? 1.0 : 2.5);
         LQ_ABORT_IF(((nm[j] | dm[j]) >> n) != 0, "operation acts on a wire outside the state");
         const bool dot = ops[j].is_dot();
         auto dep = [&](int i) {
@@ -1347,7 +1502,7 @@ std::vector<PassPlan> plan_passes(const std::vector<LOp> &ops, const PlanConfig 
             t.kind = o.kind;
             t.flags = o.flags;
             if (!o.is_dot() && o.is_swap()) t.flags |= TF_SWAP;
-            if (has_dots) t.flags |= o.is_dot() ? o.dot_class() : o.is_unitary() ? TF_UNITARY : 0u;
+            if (has_dots) t.flags |= o.is_dot() ? o.dot_class() : !cfg.keep_grouping && o.is_unitary() ? TF_UNITARY : 0u;
             t.k = static_cast<uint32_t>(o.k);
             t.smask = o.smask;
             t.sa = o.sa;
@@ -1396,10 +1551,12 @@ std::vector<PassPlan> plan_passes(const std::vector<LOp> &ops, const PlanConfig 
 
 std::string plan_structure_key(const std::vector<LOp> &ops, const PlanConfig &cfg) {
     std::string key;
+    key.reserve(ops.size() * 32 + 128);
     auto put = [&key](const void *p, size_t n) { key.append(static_cast<const char *>(p), n); };
     const double b = cfg.budget;
-    const int32_t hdr[9] = {cfg.n, cfg.ns, cfg.kt_max, cfg.low_bits, cfg.reg_rb, cfg.max_dots,
-                            cfg.scale_rotations ? 1 : 0, cfg.lookahead ? 1 : 0, cfg.dense_passes ? 1 : 0};
+    const int32_t hdr[10] = {cfg.n, cfg.ns, cfg.kt_max, cfg.low_bits, cfg.reg_rb, cfg.max_dots,
+                             cfg.scale_rotations ? 1 : 0, cfg.lookahead ? 1 : 0, cfg.dense_passes ? 1 : 0,
+                             cfg.keep_grouping ? 1 : 0};
     put(hdr, sizeof(hdr));
     put(&b, sizeof(b));
     put(&cfg.first_budget, sizeof(cfg.first_budget));
@@ -1418,13 +1575,21 @@ std::string plan_structure_key(const std::vector<LOp> &ops, const PlanConfig &cf
             else if (o.k == 0 && o.coef.size() == 1 && o.coef[0] == mone) vflags = 3;
         }
         if (has_dots) vflags |= o.is_dot() ? o.dot_class() : o.is_unitary() ? TF_UNITARY : 0u;
-        const uint32_t w[8] = {o.kind, o.flags, static_cast<uint32_t>(o.k), o.smask, o.sa, o.sb,
-                               static_cast<uint32_t>(o.slot), vflags};
+        // fields that are zero for most ops are written only where they are
+        // not, behind a byte that says which
+        const uint64_t m[8] = {o.cmask, o.cval, o.xmask, o.yzmask, o.pmask, o.pc_dim, static_cast<uint64_t>(o.ny),
+                               (static_cast<uint64_t>(o.sa) << 32) | o.sb};
+        uint32_t present = 0;
+        for (int j = 0; j < 8; ++j) present |= (m[j] != 0 ? 1u : 0u) << j;
+        const uint32_t w[5] = {o.kind | (static_cast<uint32_t>(o.k) << 8) | (o.smask << 16) | (present << 24), o.flags,
+                               vflags, static_cast<uint32_t>(o.slot), static_cast<uint32_t>(o.coef.size())};
         put(w, sizeof(w));
-        put(o.bits, sizeof(int) * static_cast<size_t>(std::max(0, std::min(o.k, kMaxTileOpTargets))));
-        const uint64_t m[7] = {o.cmask, o.cval, o.xmask, o.yzmask, o.pmask, o.pc_dim,
-                               static_cast<uint64_t>(o.coef.size()) | (static_cast<uint64_t>(o.ny) << 32)};
-        put(m, sizeof(m));
+        int8_t b8[kMaxTileOpTargets];
+        const int nb = std::max(0, std::min(o.k, kMaxTileOpTargets));
+        for (int j = 0; j < nb; ++j) b8[j] = static_cast<int8_t>(o.bits[j]);
+        put(b8, static_cast<size_t>(nb));
+        for (int j = 0; j < 8; ++j)
+            if (m[j]) put(&m[j], sizeof(uint64_t));
     }
     return key;
 }

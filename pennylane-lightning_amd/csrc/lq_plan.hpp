@@ -70,8 +70,9 @@ bool try_merge_1q(std::vector<LOp> &queue, const LOp &op);
 // (the Z-Y-Z Euler form, global phase folded into the last factor). Register
 // passes then apply the rotation with real arithmetic and apply the phases of
 // a stage's register bits together as one table (TOP_RPHASE). Gates whose
-// factors do not reproduce U to 1e-13 are kept whole.
-void split_1q_rotations(std::vector<LOp> &prog);
+// factors do not reproduce U to 1e-13 are kept whole. keep_grouping: see
+// PlanConfig.
+void split_1q_rotations(std::vector<LOp> &prog, bool keep_grouping = false);
 
 // The state before `prog` is the product state with amplitude
 // prod_q f[2q + bit q of the index] (f holds one pair per physical bit).
@@ -143,6 +144,12 @@ struct PlanConfig {
     // dense operators on three to six bits (not dots) run in passes of their
     // own on the matrix cores instead of as LDS ops of a tile pass
     bool dense_passes = false;
+    // complex64: factors of 2x2 gates by Euler angles, phases grouped between
+    // dots only and X and SWAP at a dense op's cost in the budget, as the
+    // passes of single-precision states always were. Another grouping moves
+    // every amplitude by rounding, and expectation values, which come back in
+    // double precision, by some 1e-7 of their size.
+    bool keep_grouping = false;
     // choose each pass's tile bits by lookahead (the bits that let the most
     // work run) instead of taking the first ready op's bits
     bool lookahead = false;

@@ -9,6 +9,7 @@ from __future__ import annotations
 import atexit
 import ctypes as C
 import os
+from array import array
 
 import numpy as np
 
@@ -145,11 +146,14 @@ def check(rc: int) -> None:
 
 
 def u32(xs):
-    a = np.ascontiguousarray(np.asarray(list(xs), dtype=np.uint32).reshape(-1))
-    if a.size == 0:
-        a = np.zeros(1, dtype=np.uint32)
-        return a, a.ctypes.data_as(_U32P), 0
-    return a, a.ctypes.data_as(_U32P), a.size
+    try:
+        a = array("I", xs)
+    except (TypeError, ValueError):  # floats, nested lists, tensors
+        a = array("I", np.ascontiguousarray(np.asarray(list(xs), dtype=np.uint32).reshape(-1)).tolist())
+    n = len(a)
+    if n == 0:
+        a.append(0)
+    return a, C.cast(a.buffer_info()[0], _U32P), n
 
 
 def u8(xs):

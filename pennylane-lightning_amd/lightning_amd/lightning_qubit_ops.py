@@ -27,6 +27,8 @@ from __future__ import annotations
 import ctypes as C
 import sys
 import types
+from array import array
+from itertools import accumulate, chain
 from typing import Sequence
 
 import numpy as np
@@ -358,21 +360,14 @@ class _StateVectorBase:
                                      "must all be equal")
         if n == 0:
             return
-        blob = b"\0".join(_name_bytes(o) for o in ops) + b"\0"
-        woff = np.zeros(n + 1, dtype=np.uint32)
-        np.cumsum([len(w) for w in wires], out=woff[1:])
-        wflat = np.fromiter((x for w in wires for x in w), dtype=np.uint32, count=int(woff[-1]))
-        inv = np.fromiter((1 if x else 0 for x in inverses), dtype=np.uint8, count=n)
-        pp = pf = None
+        blob = b"\0".join(map(_NAME_BYTES.__getitem__, ops)) + b"\0"
+        woff, wflat = _flatten("I", wires)
+        inv = _flags(inverses)
+        poff = pfl = None
         if params is not None:
-            poff = np.zeros(n + 1, dtype=np.uint32)
-            np.cumsum([len(p) for p in params], out=poff[1:])
-            pfl = np.fromiter((x for p in params for x in p), dtype=np.float64, count=int(poff[-1]))
-            pp = poff.ctypes.data_as(C.POINTER(C.c_uint32))
-            pf = pfl.ctypes.data_as(C.POINTER(C.c_double))
-        check(lib.lq_sv_apply_operations(self._h, n, blob, woff.ctypes.data_as(C.POINTER(C.c_uint32)),
-                                         wflat.ctypes.data_as(C.POINTER(C.c_uint32)),
-                                         inv.ctypes.data_as(C.POINTER(C.c_uint8)), pp, pf))
+            poff, pfl = _flatten("d", params)
+        check(lib.lq_sv_apply_operations(self._h, n, blob, _addr(woff, C.c_uint32), _addr(wflat, C.c_uint32),
+                                         _addr(inv, C.c_uint8), _addr(poff, C.c_uint32), _addr(pfl, C.c_double)))
 
     def applyMatrix(self, matrix, wires, inverse=False):
         m = np.ascontiguousarray(np.asarray(matrix, dtype=self._cdtype).reshape(-1))
@@ -444,14 +439,54 @@ class _StateVectorBase:
         check(lib.lq_sv_apply_ops(self._h, ops._h, int(bool(adjoint))))
 
 
-_NAME_BYTES = {}
+class _NameBytes(dict):
+    """Encoded gate names."""
+
+    def __missing__(self, name):
+        b = self[name] = name.encode()
+        return b
+
+
+_NAME_BYTES = _NameBytes()
 
 
 def _name_bytes(name: str) -> bytes:
-    b = _NAME_BYTES.get(name)
-    if b is None:
-        b = _NAME_BYTES[name] = name.encode()
-    return b
+    return _NAME_BYTES[name]
+
+
+def _flatten(code, lists):
+    """Offsets (uint32, one more than lists) and the concatenated values of
+    type ``code`` (array module)."""
+    try:
+        off = array("I", accumulate(map(len, lists), initial=0))
+    except TypeError:  # iterators
+        lists = [list(v) for v in lists]
+        off = array("I", accumulate(map(len, lists), initial=0))
+    try:
+        return off, array(code, chain.from_iterable(lists))
+    except TypeError:  # values that only convert explicitly (a float standing for a wire)
+        conv = float if code == "d" else int
+        return off, array(code, [conv(x) for v in lists for x in v])
+
+
+def _first(lists, n):
+    """The first n entries; fewer are an error, as indexing them would be."""
+    if len(lists) < n:
+        raise IndexError("list index out of range")
+    return lists if len(lists) == n else lists[:n]
+
+
+def _flags(values):
+    """Truth values as bytes."""
+    try:
+        return array("B", values)
+    except (TypeError, OverflowError, ValueError):
+        return array("B", [1 if v else 0 for v in values])
+
+
+def _addr(a, ctype):
+    """An array's data as a ctypes pointer (None: null)."""
+    return None if a is None else C.cast(a.buffer_info()[0], C.POINTER(ctype))
 
 
 def _make_gate(name):
@@ -749,48 +784,64 @@ class MeasurementsC128(_MeasurementsBase):
 # ---------------------------------------------------------------------------
 # Algorithms (core/algorithms/JacobianData.hpp, lq/algorithms/AdjointJacobianLQubit.hpp)
 # ---------------------------------------------------------------------------
+_NO_MATRIX = np.zeros(0, np.complex128)
+
+
 class OpsStruct:
     """OpsData: names, params, wires, inverses, matrices[, ctrl wires, ctrl values]."""
 
     def __init__(self, ops_name, ops_params, ops_wires, ops_inverses, ops_matrices,
                  ops_controlled_wires=None, ops_controlled_values=None):
         n = len(ops_name)
-        ops_controlled_wires = ops_controlled_wires or [[] for _ in range(n)]
-        ops_controlled_values = ops_controlled_values or [[] for _ in range(n)]
+        none = [()] * n
+        ops_controlled_wires = ops_controlled_wires or none
+        ops_controlled_values = ops_controlled_values or none
         self.names = list(ops_name)
-        self.params = [list(map(float, p)) for p in ops_params]
-        self.wires = [list(map(int, w)) for w in ops_wires]
-        self.inverses = [bool(i) for i in ops_inverses]
-        self.matrices = [np.asarray(m, dtype=np.complex128).reshape(-1) if m is not None and len(m) else
-                         np.zeros(0, np.complex128) for m in ops_matrices]
-        self.ctrl_wires = [list(map(int, c)) for c in ops_controlled_wires]
-        self.ctrl_values = [list(map(bool, v)) for v in ops_controlled_values]
-        poff, woff, moff, coff = [0], [0], [0], [0]
-        params, wires, mats, ctrls, cvals = [], [], [], [], []
-        for i in range(n):
-            params += self.params[i]
-            poff.append(len(params))
-            wires += self.wires[i]
-            woff.append(len(wires))
-            m = self.matrices[i]
-            mats += [x for z in m for x in (z.real, z.imag)]
-            moff.append(len(mats) // 2)
-            ctrls += self.ctrl_wires[i]
-            cvals += self.ctrl_values[i]
-            coff.append(len(ctrls))
-        keep = [np.asarray(poff, np.uint32), np.asarray(params + [0.0], np.float64),
-                np.asarray(woff, np.uint32), np.asarray(wires + [0], np.uint32),
-                np.asarray([int(b) for b in self.inverses] + [0], np.uint8), np.asarray(moff, np.uint32),
-                np.asarray(mats + [0.0], np.float64), np.asarray(coff, np.uint32),
-                np.asarray(ctrls + [0], np.uint32), np.asarray([int(b) for b in cvals] + [0], np.uint8)]
-        names = (C.c_char_p * max(n, 1))(*[s.encode() for s in self.names])
-        ptr = lambda a, t: a.ctypes.data_as(C.POINTER(t))
+        self.inverses = list(map(bool, ops_inverses))
+        self.matrices = [_NO_MATRIX if m is None or not len(m) else np.asarray(m, dtype=np.complex128).reshape(-1)
+                         for m in _first(ops_matrices, n)]
+        # flat copies, as the engine takes them; ``params``, ``wires`` and the
+        # controls are read back from them
+        self._params = poff, params = _flatten("d", _first(ops_params, n))
+        self._wires = woff, wires = _flatten("I", _first(ops_wires, n))
+        self._ctrls = coff, ctrls = _flatten("I", _first(ops_controlled_wires, n))
+        if ops_controlled_values is not none:
+            ops_controlled_values = [[1 if v else 0 for v in vs] for vs in _first(ops_controlled_values, n)]
+        self._cvals_off, self._cvals = _flatten("B", ops_controlled_values)
+        moff = array("I", accumulate(map(len, self.matrices), initial=0))
+        mats = [m for m in self.matrices if m is not _NO_MATRIX]
+        flat = np.ascontiguousarray(np.concatenate(mats) if mats else np.zeros(1, np.complex128))
+        inv = array("B", (self.inverses + [False] * n)[:n] + [False])
+        cvals = self._cvals + array("B", bytes(max(0, len(ctrls) - len(self._cvals)) + 1))
+        names = (C.c_char_p * max(n, 1))(*map(_NAME_BYTES.__getitem__, self.names))
+        zero = array("d", [0.0])  # stands for empty arrays
         h = C.c_void_p()
-        check(lib.lq_ops_create(n, names, ptr(keep[0], C.c_uint32), ptr(keep[1], C.c_double),
-                                ptr(keep[2], C.c_uint32), ptr(keep[3], C.c_uint32), ptr(keep[4], C.c_uint8),
-                                ptr(keep[5], C.c_uint32), ptr(keep[6], C.c_double), ptr(keep[7], C.c_uint32),
-                                ptr(keep[8], C.c_uint32), ptr(keep[9], C.c_uint8), C.byref(h)))
+        check(lib.lq_ops_create(n, names, _addr(poff, C.c_uint32), _addr(params or zero, C.c_double),
+                                _addr(woff, C.c_uint32), _addr(wires or zero, C.c_uint32), _addr(inv, C.c_uint8),
+                                _addr(moff, C.c_uint32), flat.ctypes.data_as(C.POINTER(C.c_double)),
+                                _addr(coff, C.c_uint32), _addr(ctrls or zero, C.c_uint32),
+                                _addr(cvals, C.c_uint8), C.byref(h)))
         self._h = h
+
+    @staticmethod
+    def _lists(off, values):
+        return [list(values[off[i]:off[i + 1]]) for i in range(len(off) - 1)]
+
+    @property
+    def params(self):
+        return self._lists(*self._params)
+
+    @property
+    def wires(self):
+        return self._lists(*self._wires)
+
+    @property
+    def ctrl_wires(self):
+        return self._lists(*self._ctrls)
+
+    @property
+    def ctrl_values(self):
+        return [[bool(v) for v in vs] for vs in self._lists(self._cvals_off, self._cvals)]
 
     def __del__(self):
         h = getattr(self, "_h", None)
@@ -824,7 +875,7 @@ class Recording:
         check(lib.lq_sv_record(sv._h, operations._h, C.byref(h)))
         self._h = h
         self._sv = sv
-        self.nparams = sum(len(p) for p in operations.params)
+        self.nparams = len(operations._params[1])
 
     def replay(self, params):
         p = np.ascontiguousarray(np.asarray(params, dtype=np.float64).reshape(-1))

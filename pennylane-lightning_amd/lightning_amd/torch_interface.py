@@ -48,18 +48,21 @@ def adjoint_form(ops):
 def bind(ops, values):
     """Copy of ``ops`` with the parameters of the parametric ops replaced, in order."""
     it = iter(np.asarray(values, dtype=np.float64).tolist())
-    out = []
-    for op in ops:
-        if op.params:
-            out.append(CircuitOp(op.name, op.wires, [next(it) for _ in op.params], op.inverse, op.matrix,
-                                 op.ctrls, op.cvals))
-        else:
-            out.append(op)
-    return out
+
+    def bound(op):
+        out = object.__new__(CircuitOp)
+        out.__dict__.update(op.__dict__)
+        out.params = [next(it) for _ in op.params]
+        return out
+
+    return [bound(op) if op.params else op for op in ops]
 
 
 def num_params(ops) -> int:
     return sum(len(op.params) for op in ops)
+
+
+_ONE_WIRE = frozenset(("PauliX", "PauliY", "PauliZ", "Hadamard", "Identity"))
 
 
 class _CircuitExpvals(torch.autograd.Function):
@@ -70,7 +73,12 @@ class _CircuitExpvals(torch.autograd.Function):
         sv = (L.StateVectorC128 if bits == 128 else L.StateVectorC64)(n)
         apply_circuit(sv, bound)
         m = (L.MeasurementsC128 if bits == 128 else L.MeasurementsC64)(sv)
-        ev = np.array([m.expval(observable(o, bits)) for o in observables], dtype=np.float64)
+        if bits == 128 and len(observables) > 1 and all(o[0] == "N" and o[1] in _ONE_WIRE for o in observables):
+            # one program for the circuit and all of them (in single precision
+            # another set of dots means other passes and another rounding)
+            ev = m.expval_named_batch([o[1] for o in observables], [o[2] for o in observables])
+        else:
+            ev = np.array([m.expval(observable(o, bits)) for o in observables], dtype=np.float64)
         ctx.sv, ctx.bound, ctx.observables, ctx.bits = sv, bound, observables, bits
         ctx.param_dtype, ctx.param_device = params.dtype, params.device
         return torch.as_tensor(ev, dtype=params.dtype, device=params.device)

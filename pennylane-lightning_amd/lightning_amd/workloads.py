@@ -8,6 +8,8 @@ from __future__ import annotations
 
 import math
 from dataclasses import dataclass, field
+from itertools import repeat
+from operator import attrgetter, is_
 
 import numpy as np
 
@@ -132,23 +134,33 @@ def qft_brickwork_mcx(n: int, layers: int = 8, mcx_per_layer: int = 1, seed: int
     return ops
 
 
+_MATRIX, _CTRLS = attrgetter("matrix"), attrgetter("ctrls")
+
+
+def _all_none(values) -> bool:
+    return all(map(is_, values, repeat(None)))
+
+
 def apply_circuit(sv, ops: list[CircuitOp]) -> None:
     """Apply an op list to a StateVectorC*: runs of plain named gates with
     one ``applyOperations`` call each, matrices and controlled gates through
     their own methods."""
-    run = []
+    fields = attrgetter("name", "wires", "inverse", "params")
 
-    def flush_run():
+    def run_plain(run):
         if run:
-            sv.applyOperations([o.name for o in run], [o.wires for o in run], [o.inverse for o in run],
-                               [o.params for o in run])
-            run.clear()
+            sv.applyOperations(*zip(*map(fields, run)))
 
-    for op in ops:
+    ops = ops if isinstance(ops, (list, tuple)) else list(ops)
+    if _all_none(map(_MATRIX, ops)) and not any(map(_CTRLS, ops)):
+        run_plain(ops)
+        return
+    start = 0
+    for i, op in enumerate(ops):
         if op.matrix is None and not op.ctrls:
-            run.append(op)
             continue
-        flush_run()
+        run_plain(ops[start:i])
+        start = i + 1
         if op.matrix is not None:
             if op.ctrls:
                 sv.applyControlledMatrix(op.matrix, op.ctrls, op.cvals or [True] * len(op.ctrls), op.wires,
@@ -157,16 +169,18 @@ def apply_circuit(sv, ops: list[CircuitOp]) -> None:
                 sv.applyMatrix(op.matrix, op.wires, op.inverse)
         else:
             getattr(sv, op.name)(op.ctrls, op.cvals or [True] * len(op.ctrls), op.wires, op.inverse, op.params)
-    flush_run()
+    run_plain(ops[start:])
 
 
 def to_ops(ops: list[CircuitOp], bits: int = 128):
     """OpsStructC64/C128 of an op list (the adjoint Jacobian's input)."""
     from . import lightning_qubit_ops as L
     cls = L.OpsStructC128 if bits == 128 else L.OpsStructC64
-    return cls([o.name for o in ops], [o.params for o in ops], [o.wires for o in ops], [o.inverse for o in ops],
-               [o.matrix if o.matrix is not None else [] for o in ops], [o.ctrls for o in ops],
-               [o.cvals or [True] * len(o.ctrls) for o in ops])
+    ops = ops if isinstance(ops, (list, tuple)) else list(ops)
+    names, params, wires, inverses, matrices, ctrls = (
+        zip(*map(attrgetter("name", "params", "wires", "inverse", "matrix", "ctrls"), ops)) if ops else [()] * 6)
+    cvals = [o.cvals or [True] * len(o.ctrls) for o in ops] if any(ctrls) else None
+    return cls(names, params, wires, inverses, matrices, ctrls if cvals else None, cvals)
 
 
 def hamiltonian_obs(coeffs, words, bits: int = 128):
