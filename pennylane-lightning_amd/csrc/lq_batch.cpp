@@ -138,21 +138,24 @@ constexpr size_t kRunnerOutBytes = 1u << 20;
 constexpr size_t kSectionAlign = 256; // each of the 5 sections starts 256-byte aligned
 } // namespace
 
-BatchRunner::BatchRunner() {
-    // a hardware queue of its own: a CU-masked stream (every CU enabled) gets
-    // a new queue instead of sharing one with other streams once the
-    // process's queue pool is full, where it would wait behind their kernels
+hipStream_t own_queue_stream() {
     int dev = 0, cus = 0;
     const char *oq = std::getenv("LQ_BATCH_OWN_QUEUE");
+    if (oq && std::atoi(oq) == 0) return nullptr;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+        return nullptr;
+    std::vector<uint32_t> mask((static_cast<size_t>(cus) + 31) / 32, 0u);
+    for (int c = 0; c < cus; ++c) mask[static_cast<size_t>(c) / 32] |= 1u << (c % 32);
+    hipStream_t s = nullptr;
+    if (hipExtStreamCreateWithCUMask(&s, static_cast<uint32_t>(mask.size()), mask.data()) != hipSuccess) return nullptr;
+    return s;
+}
+
+BatchRunner::BatchRunner() {
     const char *ku = std::getenv("LQ_BATCH_KERNEL_UPLOAD");
     kernel_upload_ = !ku || std::atoi(ku) != 0;
-    if ((!oq || std::atoi(oq) != 0) && hipGetDevice(&dev) == hipSuccess &&
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus > 0) {
-        std::vector<uint32_t> mask((static_cast<size_t>(cus) + 31) / 32, 0u);
-        for (int c = 0; c < cus; ++c) mask[static_cast<size_t>(c) / 32] |= 1u << (c % 32);
-        if (hipExtStreamCreateWithCUMask(&stream_, static_cast<uint32_t>(mask.size()), mask.data()) != hipSuccess)
-            stream_ = nullptr;
-    }
+    stream_ = own_queue_stream();
     if (!stream_) hip_check(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking), "hipStreamCreate");
     hip_check(hipEventCreateWithFlags(&done_, hipEventDisableTiming), "hipEventCreate");
     for (hipEvent_t *e : {&t0_, &t_in_, &t_k_, &t_out_}) hip_check(hipEventCreate(e), "hipEventCreate");
