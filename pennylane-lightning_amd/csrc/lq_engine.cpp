@@ -797,6 +797,11 @@ StateVector::Planned StateVector::plan(const std::vector<LOp> &prog, int ns, boo
     // a state that is one tile gains nothing from a second pass (complex64
     // keeps its passes with its grouping)
     if (t.budget <= 0 && n_ <= cfg.kt_max && dtype_) cfg.budget = 1e9;
+    // states whose passes are never specialised: a pass of a few workgroups
+    // costs 8 us besides its ops (launch, program, tile in and out), so fewer
+    // and longer ones (gradient of 13 qubits, two states: 24 -> 1030 us, 32 ->
+    // 970, 56 -> 944, 80 -> 922, 120 -> 921)
+    else if (t.budget <= 0 && n_ < jit_config().min_qubits && dtype_) cfg.budget = 80.0;
     // register-resident passes for tiles of 11 or 12 bits with one or two states
     const int ktr = std::min(cfg.kt_max, 8 + kMaxRegBits);
     if (t.reg && ns <= 2 && n_ >= 11 && ktr >= 11) {

@@ -66,6 +66,26 @@ template <int NS, typename F> __device__ __forceinline__ void with_pair(uint32_t
     }
 }
 
+// Dots with X, Y or Z of which one part is used, between the states of an
+// adjoint sweep (two states, imaginary part) or of one state with itself (real
+// part): two FMAs an amplitude and one wave sum in place of 12 and two. A
+// narrow workgroup of four waves is bound by instruction issue (13 qubits, two
+// states: 260 vector instructions an op, half of the ops dots).
+template <int NS> __device__ __forceinline__ bool class_dot(const OpView &op, uint32_t cls) {
+    return (op.flags() & cls) && (op.flags() & (NS == 2 ? TF_DOT_IM : TF_DOT_RE)) && op.sa() == 0 && op.sb() == NS - 1 &&
+           op.gcmask() == 0;
+}
+// the part of conj(b) v
+template <int NS, typename V> __device__ __forceinline__ double dot_part(V b, V v) {
+    const double bx = b.x, by = b.y, vx = v.x, vy = v.y;
+    return NS == 2 ? bx * vy - by * vx : bx * vx + by * vy;
+}
+// the part of conj(b) i v
+template <int NS, typename V> __device__ __forceinline__ double dot_part_i(V b, V v) {
+    const double bx = b.x, by = b.y, vx = v.x, vy = v.y;
+    return NS == 2 ? bx * vx + by * vy : by * vx - bx * vy;
+}
+
 // One-bit phase diag(d0, d1), no controls, on register bit I of the stage.
 template <typename T, int NS, int RB, int I>
 __device__ __forceinline__ void reg_phase_reg(Regs<T, NS, RB> &R, const OpView &op, typename VecT<T>::type d0,
@@ -117,6 +137,21 @@ __device__ __forceinline__ void reg_dense1(Regs<T, NS, RB> &R, const OpView &op,
     const V m10 = op.template c<T>(2), m11 = op.template c<T>(3);
     const uint64_t gcm = op.gcmask(), gcv = op.gcval();
     if (op.flags() & TF_DOT) {
+        if (class_dot<NS>(op, TF_DOT_X | TF_DOT_Y)) {
+            double acc = 0.0;
+            if (op.flags() & TF_DOT_X) {
+#pragma unroll
+                for (int e = 0; e < E; ++e) acc += dot_part<NS>(R.v[NS - 1][e], R.v[0][e ^ (1 << I)]);
+            } else {
+#pragma unroll
+                for (int e = 0; e < E; ++e) {
+                    const double q = dot_part_i<NS>(R.v[NS - 1][e], R.v[0][e ^ (1 << I)]);
+                    acc += ((e >> I) & 1) ? q : -q;
+                }
+            }
+            (NS == 2 ? acci : accr) = acc;
+            return;
+        }
         with_pair<NS>(op.sa(), op.sb(), [&](auto A, auto B) {
             constexpr int sa = decltype(A)::value, sb = decltype(B)::value;
 #pragma unroll
@@ -305,6 +340,17 @@ __device__ __forceinline__ void reg_diag(Regs<T, NS, RB> &R, const OpView &op, c
 #pragma unroll
         for (int i = 0; i < RB; ++i)
             if (rg[i] == b) r = i;
+        if ((op.flags() & TF_DOT) && class_dot<NS>(op, TF_DOT_Z)) {
+            double acc = 0.0;
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                const double q = dot_part<NS>(R.v[NS - 1][e], R.v[0][e]);
+                const uint32_t neg = r < 0 ? 0u : (static_cast<uint32_t>(e) >> r) & 1u; // uniform
+                acc += __hiloint2double(__double2hiint(q) ^ static_cast<int>(neg << 31), __double2loint(q));
+            }
+            (NS == 2 ? acci : accr) = r < 0 && (gbt & b) ? -acc : acc;
+            return;
+        }
         switch (r) {
         case 0: reg_phase_reg<T, NS, RB, 0>(R, op, d0, d1, accr, acci); return;
         case 1: if constexpr (RB > 1) reg_phase_reg<T, NS, RB, 1>(R, op, d0, d1, accr, acci); return;
@@ -500,7 +546,9 @@ __global__ __launch_bounds__(kBlock) void tile_reg_kernel(TileRegArgs a, typenam
                 double accr = 0.0, acci = 0.0;
                 reg_apply<T, NS, RB, WIDE>(R, op, ops[oi], coef, gbt, rg, accr, acci);
                 if (op.flags() & TF_DOT) {
-                    wave_sum(accr, acci);
+                    // the part that is not used is left as this wave's first lane has it
+                    if (!(op.flags() & TF_DOT_IM)) accr = wave_sum1(accr);
+                    if (!(op.flags() & TF_DOT_RE)) acci = wave_sum1(acci);
                     if ((tid & 63u) == 0) dred[tid >> 6][op.slot()] = make_double2(accr, acci);
                 }
             }
