@@ -240,6 +240,88 @@ __global__ __launch_bounds__(kBlock) void pauli_sum_kernel(const typename VecT<T
     if (MODE == 0) block_reduce_store(energy, 0.0, red, &partials[blockIdx.x]);
 }
 
+// The same sum of P_t a for large complex128 states. pauli_sum_kernel reads the
+// state once for each x through the L2 (13 TB/s of mostly misses); here a
+// workgroup brings a tile of 2^12 amplitudes (its own ^ the high bits of x) to
+// LDS once for all terms that share those bits and takes a[i ^ x] from there,
+// the next group's tile in flight meanwhile, its sums in registers (8
+// amplitudes a thread, in the order of the terms as there); two workgroups of
+// 64 KiB a CU. 24 qubits, 200 random words in 136 groups: 4.43 -> 3.40 ms (10.7
+// TB/s). Groups of many terms are bound by the LDS reads instead, where the L1
+// does as well.
+__global__ __launch_bounds__(kPauliTileThreads) void pauli_tile_kernel(const double2 *__restrict__ a,
+                                                                      double2 *__restrict__ out,
+                                                                      const PauliTerm *__restrict__ terms,
+                                                                      const uint32_t *__restrict__ ends,
+                                                                      uint32_t ngroups, uint64_t ntiles) {
+    using T = double;
+    using V = double2;
+    constexpr int U = (1 << kPauliTileBits) / kPauliTileThreads;
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    V *lds = reinterpret_cast<V *>(smem_raw);
+    const uint32_t tid = threadIdx.x;
+    KTerm *kt = (KTerm *)terms;
+    typedef __attribute__((address_space(4))) const uint32_t KEnd;
+    KEnd *ke = (KEnd *)ends;
+    // XCD b % 8 takes an eighth of the tiles in order: its workgroups read
+    // neighbouring tiles at a time (ntiles is a power of two, at least 8)
+    const uint64_t tile = (blockIdx.x & 7ull) * (ntiles >> 3) + (blockIdx.x >> 3);
+    const uint64_t base = tile << kPauliTileBits;
+    T px[U], py[U]; // the tile in flight
+    double sr[U], si[U];
+    auto fetch = [&](uint64_t x) {
+        const V *src = a + (base ^ (x >> kPauliTileBits << kPauliTileBits));
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const V v = src[u * kPauliTileThreads + tid];
+            px[u] = v.x;
+            py[u] = v.y;
+        }
+    };
+#pragma unroll
+    for (int u = 0; u < U; ++u) sr[u] = si[u] = 0.0;
+    fetch(kt[0].x);
+    uint32_t t = 0;
+    for (uint32_t g = 0; g < ngroups; ++g) {
+        const uint32_t end = ke[g];
+        __syncthreads(); // the last group's reads
+#pragma unroll
+        for (int u = 0; u < U; ++u) lds[u * kPauliTileThreads + tid] = mk<T>(px[u], py[u]);
+        __syncthreads();
+        if (g + 1 < ngroups) fetch(kt[end].x);
+        for (; t < end; ++t) {
+            const uint64_t yz = kt[t].yz;
+            const uint32_t x = static_cast<uint32_t>(kt[t].x) & ((1u << kPauliTileBits) - 1u);
+            const double cre = kt[t].cre, cim = kt[t].cim;
+            const uint32_t sg = static_cast<uint32_t>(__popc(tid & static_cast<uint32_t>(yz))) << 31;
+            const bool real = (__double_as_longlong(cim) << 1) == 0, imag = (__double_as_longlong(cre) << 1) == 0;
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const uint32_t s = sg ^ (static_cast<uint32_t>(__popcll((base + u * kPauliTileThreads) & yz)) << 31);
+                const V v = lds[(u * kPauliTileThreads + tid) ^ x];
+                const double vx = v.x, vy = v.y;
+                auto sgn = [&](double c) { return __hiloint2double(__double2hiint(c) ^ static_cast<int>(s), __double2loint(c)); };
+                if (real) {
+                    const double c = sgn(cre);
+                    sr[u] += c * vx;
+                    si[u] += c * vy;
+                } else if (imag) {
+                    const double c = sgn(cim);
+                    sr[u] -= c * vy;
+                    si[u] += c * vx;
+                } else {
+                    const double c = sgn(cre), d = sgn(cim);
+                    sr[u] += c * vx - d * vy;
+                    si[u] += c * vy + d * vx;
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+        out[base + u * kPauliTileThreads + tid] = mk<T>(static_cast<T>(sr[u]), static_cast<T>(si[u]));
+}
+
 template <typename T>
 __global__ __launch_bounds__(kBlock) void norm2_kernel(const typename VecT<T>::type *a, uint64_t N, double2 *partials) {
     __shared__ double2 red[kBlock / 64];
@@ -617,6 +699,14 @@ template void launch_pauli_sum<double>(const void *, void *, const PauliTerm *, 
                                        hipStream_t);
 template void launch_pauli_sum<float>(const void *, void *, const PauliTerm *, uint32_t, int, int, double2 *,
                                       hipStream_t);
+
+void launch_pauli_tiles(const void *a, void *out, const PauliTerm *terms, const uint32_t *ends, uint32_t ngroups, int n,
+                        hipStream_t s) {
+    const uint64_t ntiles = 1ull << (n - kPauliTileBits);
+    hipLaunchKernelGGL(pauli_tile_kernel, dim3(static_cast<uint32_t>(ntiles)), dim3(kPauliTileThreads),
+                       sizeof(double2) << kPauliTileBits, s, static_cast<const double2 *>(a),
+                       static_cast<double2 *>(out), terms, ends, ngroups, ntiles);
+}
 
 template <typename T> void launch_norm2(const void *a, int n, double2 *partials, uint32_t nblocks, hipStream_t s) {
     using V = typename VecT<T>::type;

@@ -97,6 +97,15 @@ template <typename T>
 void launch_pauli_sum(const void *a, void *out, const PauliTerm *terms, uint32_t nterms, int n,
                       int mode, double2 *partials, hipStream_t s);
 
+// mode 1 on complex128 states for sorted terms in groups of equal
+// x >> kPauliTileBits; ends[g] is one past group g's last term; at least one
+// group, n >= kPauliTileBits + 3
+constexpr int kPauliTileBits = 12, kPauliTileThreads = 512;
+constexpr int kPauliTileQubits = 24;
+constexpr size_t kPauliTileTerms = 32;
+void launch_pauli_tiles(const void *a, void *out, const PauliTerm *terms, const uint32_t *ends, uint32_t ngroups, int n,
+                        hipStream_t s);
+
 // sum_i |a_i|^2 into per-block partials
 template <typename T>
 void launch_norm2(const void *a, int n, double2 *partials, uint32_t nblocks, hipStream_t s);
