@@ -157,7 +157,7 @@ int lq_probs(lq_sv_t sv, const uint32_t *wires, uint32_t nw, int all, double *ou
  * result 2^nw doubles in the caller's device memory out_dev (wires[0] the
  * most significant bit of the result index, as lq_probs), enqueued on
  * `stream` (a hipStream_t; NULL: the null stream); the caller synchronizes.
- * No allocation: the per-block partial histograms go to a fixed device array
+ * No allocation: the rows of partial sums go to a fixed device array
  * of 512 x 2^10 doubles (4 MiB, held by each GPU the library runs on until
  * the process ends), so nw is limited to 1..10; every call on a GPU shares
  * that array, and calls that overlap on one GPU race. lq_probs_noalloc_init

@@ -146,8 +146,8 @@ void launch_dense_wide(const void *in, void *out, const double2 *M, const int *b
 // W = [[Re U, -Im U], [Im U, Re U]] on the device; matrix cores; n >= 12
 void launch_dense5_c64_mfma(const void *in, void *out, const float *W, int n, hipStream_t s);
 // Probabilities of 1..kNoAllocProbsMaxWires wires of a caller-owned device
-// state into device memory `out` (2^nw doubles) on stream s, with the
-// partial histograms in a fixed device array (no allocation; calls that
+// state into device memory `out` (2^nw doubles) on stream s, with the rows
+// of partial sums in a fixed device array (no allocation; calls that
 // overlap on one GPU share it). probs_noalloc_init takes the array's address
 // on the current device (the first probs_noalloc call does it otherwise).
 constexpr int kNoAllocProbsMaxWires = 10;

@@ -261,10 +261,10 @@ void Server::large_loop(bool lane) {
     // the worker's own stream: the pooled states it takes run on it, so the
     // server's streams are its workers and packed runners only, each with a
     // hardware queue of its own (states keep their own streams while idle).
-    // Ordinary streams share four hardware queues, and kernels of one queue
-    // run one after the other: ten workers' passes of four to sixteen
-    // workgroups took 18.9 ms for 64 requests of 10 to 15 qubits, 14.8 ms on
-    // queues of their own.
+    // Ordinary streams share the process's hardware queues (four, or
+    // GPU_MAX_HW_QUEUES), and kernels of one queue run one after the other: ten
+    // workers' passes of four to sixteen workgroups took 18.9 ms for 64
+    // requests of 10 to 15 qubits on four queues, 14.8 ms on their own.
     // (If no stream can be created, requests run on the states' own streams:
     // nothing may throw out of a worker thread.)
     hipStream_t ws = own_queue_stream();
