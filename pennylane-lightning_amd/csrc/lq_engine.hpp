@@ -358,6 +358,11 @@ class StateVector {
     // hipMemcpyAsync. read_back returns once the data is in `host`.
     void upload_small(void *dev, size_t dev_cap, const void *host, size_t bytes);
     void read_back(void *host, const void *dev, size_t bytes);
+    // Where a kernel writes an answer of `bytes` that only the host reads: host
+    // memory itself for short answers (one launch less than a copy kernel,
+    // 4 us a measurement), else `dev`. read_answer waits and copies it out.
+    void *answer(DevBuf &dev, size_t bytes);
+    void read_answer(void *host, const void *answer, size_t bytes);
     std::vector<std::unique_ptr<DevBuf>> ws_;
     bool prof_ = false;
     struct Pending {
