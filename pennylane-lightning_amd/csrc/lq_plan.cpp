@@ -738,11 +738,6 @@ bool diagonal_kind(uint32_t k) {
            k == TOP_RPHASE || k == TOP_TPHASE;
 }
 
-// Order of a register stage's ops by earliest level: an op's level is one
-// more than that of the latest earlier op it does not commute with. Ops
-// commute when they act on different states, or when neither acts
-// non-diagonally on a bit the other touches. Dots and ops without a known
-// bit set keep their place relative to everything.
 // Whether a dot (register form, one or two targets) and an op may change
 // places: the op is unitary, acts on both of the dot's states, and acts
 // non-diagonally on no bit the dot touches (and the dot on none of the op's).
@@ -769,7 +764,40 @@ bool dot_commutes(const TileOp &dot, const TileOp &op) {
     return !(na & (nb | db)) && !(nb & da);
 }
 
-std::vector<int> stage_levels_order(const std::vector<TileOp> &ops) {
+// A one-bit phase on a register bit: it can stand anywhere between the ops
+// that block it, from lo (before rest[lo]) to hi.
+struct RegPhase {
+    int lo, hi, r;
+    uint32_t sm;
+    cd d0, d1;
+    int at; // it stood before rest[at]
+    uint64_t src;
+    bool unit;
+};
+
+bool blocks_phase(const TileOp &l, const RegPhase &ph) {
+    if (l.flags & TF_DOT) {
+        // <b|D^dagger G D|a> = <b|G|a> for a unitary phase D on both states and
+        // a bit that G acts on diagonally or not at all
+        const uint32_t ab = (1u << l.sa) | (1u << l.sb);
+        if (!ph.unit || (ph.sm & ab) != ab) return true;
+    } else if (!(l.smask & ph.sm)) {
+        return false;
+    }
+    if (diagonal_kind(l.kind)) return false;
+    if (l.kind == TOP_DENSE1) return l.lpos[0] == ph.r;
+    if (l.kind == TOP_DENSE2) return l.lpos[0] == ph.r || l.lpos[1] == ph.r;
+    return true;
+}
+
+// Order of a register stage's ops by earliest level: an op's level is one
+// more than that of the latest earlier op it does not commute with. Ops
+// commute when they act on different states, or when neither acts
+// non-diagonally on a bit the other touches; dots commute with each other and
+// with the ops of dot_commutes, unless a phase stands between two of them that
+// neither may pass. Ops without a known bit set keep their place relative to
+// everything.
+std::vector<int> stage_levels_order(const std::vector<TileOp> &ops, const std::vector<RegPhase> &phases) {
     const int M = static_cast<int>(ops.size());
     const uint64_t ALL = ~0ull;
     std::vector<uint64_t> nd(static_cast<size_t>(M)), dg(static_cast<size_t>(M));
@@ -803,9 +831,20 @@ std::vector<int> stage_levels_order(const std::vector<TileOp> &ops) {
         return !(nd[x] & (nd[y] | dg[y])) && !(nd[y] & (nd[x] | dg[x]));
     };
     std::vector<int> level(static_cast<size_t>(M), 0);
-    for (int y = 0; y < M; ++y)
+    // of each phase, the highest level among the ops before it that block it:
+    // no op after it that blocks it may get a lower one (ops of one level keep
+    // their order)
+    std::vector<int> floor(phases.size(), 0);
+    size_t passed = 0; // phases before op y (they are in the order of their places)
+    for (int y = 0; y < M; ++y) {
+        for (; passed < phases.size() && phases[passed].at <= y; ++passed)
+            for (int x = 0; x < phases[passed].at; ++x)
+                if (level[x] > floor[passed] && blocks_phase(ops[x], phases[passed])) floor[passed] = level[x];
         for (int x = 0; x < y; ++x)
             if (!commute(x, y)) level[y] = std::max(level[y], level[x] + 1);
+        for (size_t j = 0; j < passed; ++j)
+            if (floor[j] > level[y] && blocks_phase(ops[y], phases[j])) level[y] = floor[j];
+    }
     std::vector<int> perm(static_cast<size_t>(M));
     for (int x = 0; x < M; ++x) perm[x] = x;
     std::stable_sort(perm.begin(), perm.end(), [&](int x, int y) { return level[x] < level[y]; });
@@ -814,7 +853,8 @@ std::vector<int> stage_levels_order(const std::vector<TileOp> &ops) {
 
 // In a register stage the non-diagonal ops act on register bits only, so a
 // one-bit phase on any other bit (a thread or outside bit: fixed per thread)
-// commutes with every op of the stage but a dot or an op of unknown action.
+// commutes with every op of the stage but one of unknown action and, where it
+// is not unitary or acts on one of the dot's states only, a dot.
 // Between two such blockers, the phases of one state set become one
 // TOP_TPHASE op at the first one's place: each thread forms the product of
 // their factors once and multiplies its amplitudes once, instead of once per
@@ -887,8 +927,8 @@ void group_thread_phases(PassPlan &p, std::vector<TileOp> &ops, const int *ridx)
 
 // In each register stage, one-bit phases on register bits commute with
 // diagonal ops and with dense ops on other register bits, so each can sit
-// anywhere between the ops that block it (a dense op on its bit, a dot, any
-// other non-diagonal op). Choose the fewest points that every phase's range
+// anywhere between the ops that block it (blocks_phase: a dense op or dot on
+// its bit, any dot for a phase that is not unitary, any other non-diagonal op). Choose the fewest points that every phase's range
 // contains (interval stabbing, greedy by right end) and replace the phases at
 // each point by one table over the stage's register index.
 void group_register_phases(PassPlan &p, int rb) {
@@ -906,25 +946,8 @@ void group_register_phases(PassPlan &p, int rb) {
                 return t.kind == TOP_DIAG && t.k == 1 && t.gcmask == 0 && !(t.flags & TF_DOT) && t.gpos[0] >= 0 &&
                        t.gpos[0] < 64 && ridx[t.gpos[0]] >= 0;
             };
-            auto blocks = [&](const TileOp &l, int r, uint32_t sm, bool unit) {
-                if (l.flags & TF_DOT) {
-                    // <b|D^dagger G D|a> = <b|G|a> for a phase D on both states and a
-                    // bit that G acts on diagonally or not at all
-                    const uint32_t ab = (1u << l.sa) | (1u << l.sb);
-                    if (!unit || (sm & ab) != ab) return true;
-                    if (l.kind == TOP_DENSE1) return l.lpos[0] == r;
-                    if (l.kind == TOP_DENSE2) return l.lpos[0] == r || l.lpos[1] == r;
-                    return !diagonal_kind(l.kind);
-                }
-                if (diagonal_kind(l.kind)) return false;
-                if (!(l.smask & sm)) return false;
-                if (l.kind == TOP_DENSE1) return l.lpos[0] == r;
-                if (l.kind == TOP_DENSE2) return l.lpos[0] == r || l.lpos[1] == r;
-                return true;
-            };
             std::vector<TileOp> rest;      // non-phase ops; gap g sits before rest[g]
-            struct Ph { int lo, hi, r; uint32_t sm; cd d0, d1; int at; uint64_t src; bool unit; };
-            std::vector<Ph> ph;
+            std::vector<RegPhase> ph;
             for (const TileOp &t : ops) {
                 if (is_phase(t)) {
                     ph.push_back({0, 0, ridx[t.gpos[0]], t.smask, p.coef[t.coef_off], p.coef[t.coef_off + 1],
@@ -934,28 +957,29 @@ void group_register_phases(PassPlan &p, int rb) {
                 }
             }
             const int M = static_cast<int>(rest.size());
-            // each phase's blockers (indices into rest) before and after it
-            std::vector<int> prev_b(ph.size(), -1), next_b(ph.size(), M);
-            for (size_t j = 0; j < ph.size(); ++j) {
-                for (int x = ph[j].at - 1; x >= 0; --x)
-                    if (blocks(rest[x], ph[j].r, ph[j].sm, ph[j].unit)) { prev_b[j] = x; break; }
-                for (int x = ph[j].at; x < M; ++x)
-                    if (blocks(rest[x], ph[j].r, ph[j].sm, ph[j].unit)) { next_b[j] = x; break; }
-            }
             // Reorder the other ops by their earliest level (ops that commute
             // may pass each other), so that ops on different bits at the same
             // depth sit together and the phases between them share one point.
-            std::vector<int> perm = stage_levels_order(rest);
+            std::vector<int> perm = stage_levels_order(rest, ph);
             std::vector<int> newpos(static_cast<size_t>(M));
             for (int x = 0; x < M; ++x) newpos[perm[x]] = x;
+            // a phase's range is bounded by every op that blocks it: commuting
+            // ones (two dots) may have changed places, so the nearest in program
+            // order need not be the nearest now
+            for (RegPhase &q : ph) {
+                q.lo = 0;
+                q.hi = M;
+                for (int x = 0; x < M; ++x) {
+                    if (!blocks_phase(rest[x], q)) continue;
+                    if (x < q.at) q.lo = std::max(q.lo, newpos[x] + 1);
+                    else q.hi = std::min(q.hi, newpos[x]);
+                }
+                LQ_ABORT_IF(q.lo > q.hi, "a phase between ops that changed places");
+            }
             {
                 std::vector<TileOp> re(static_cast<size_t>(M));
                 for (int x = 0; x < M; ++x) re[x] = rest[perm[x]];
                 rest.swap(re);
-            }
-            for (size_t j = 0; j < ph.size(); ++j) {
-                ph[j].lo = prev_b[j] < 0 ? 0 : newpos[prev_b[j]] + 1;
-                ph[j].hi = next_b[j] >= M ? M : newpos[next_b[j]];
             }
             std::vector<int> order(ph.size());
             for (size_t i = 0; i < ph.size(); ++i) order[i] = static_cast<int>(i);
