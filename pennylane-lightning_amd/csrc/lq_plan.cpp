@@ -1074,7 +1074,7 @@ void finish_reg_pass(PassPlan &p, int kt) {
                 slot = 0;
             }
             cur.sd[slot] = d;
-            cur.sm[slot] |= 1ull << lo;
+            cur.sm[slot] ^= 1ull << lo; // a pair that comes twice cancels
         }
         flush();
         st.op_begin = begin;
