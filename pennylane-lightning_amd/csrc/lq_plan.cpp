@@ -9,7 +9,8 @@
 // is acted on diagonally by both (controls, diagonal targets), or when both
 // are read-only dots. A pass greedily takes ready ops whose non-diagonal bits
 // fit in its tile (at most kt_max bits, the low bits always included), up to
-// a compute budget; diagonal ops fit any pass.
+// a compute budget; diagonal ops fit any pass. A dot passes only unitary ops,
+// whatever their bits: it reads every amplitude of its states.
 #include "lq_kernels.hpp"
 #include "lq_plan.hpp"
 
@@ -90,21 +91,32 @@ uint32_t LOp::dot_class() const {
     return 0;
 }
 
-bool LOp::is_unitary() const {
+bool LOp::is_unitary(double tol) const {
     if (flags & TF_ZERO_UNCTRL) return false;
-    if (kind == TOP_DIAG || kind == TOP_PARITY || kind == TOP_PCPHASE) {
+    switch (kind) {
+    case TOP_DIAG:
+    case TOP_PARITY:
+    case TOP_PCPHASE:
+    case TOP_PAULI:
         for (const cd &v : coef)
-            if (!(std::fabs(std::norm(v) - 1.0) <= 1e-12)) return false;
+            if (!(std::fabs(std::norm(v) - 1.0) <= tol)) return false;
         return true;
+    case TOP_DENSE1:
+    case TOP_DENSE2:
+    case TOP_DENSEK: break;
+    default: return false;
     }
-    if (kind != TOP_DENSE1 && kind != TOP_DENSE2) return false;
-    const size_t d = kind == TOP_DENSE1 ? 2 : 4;
-    if (coef.size() != d * d) return false;
+    const size_t d = static_cast<size_t>(1) << k;
+    if (k > kMaxUnitaryTest || coef.size() != d * d) return false;
     for (size_t a = 0; a < d; ++a)
         for (size_t b = a; b < d; ++b) {
-            cd s(a == b ? -1.0 : 0.0);
-            for (size_t r = 0; r < d; ++r) s += std::conj(coef[r * d + a]) * coef[r * d + b];
-            if (!(std::norm(s) <= 1e-24)) return false;
+            double re = a == b ? -1.0 : 0.0, im = 0.0;
+            for (size_t r = 0; r < d; ++r) {
+                const cd u = coef[r * d + a], v = coef[r * d + b];
+                re += u.real() * v.real() + u.imag() * v.imag();
+                im += u.real() * v.imag() - u.imag() * v.real();
+            }
+            if (!(re * re + im * im <= tol * tol)) return false;
         }
     return true;
 }
@@ -599,10 +611,21 @@ struct StagePlan {
     std::vector<int> ops; // indices into the program
 };
 
+// Whether a dot may be taken before or after an op that it shares no
+// non-diagonal bit with: <b|U^dagger G U|a> = <b|G|a> takes a unitary that acts
+// on both states (an op on neither does not matter to it).
+bool passes_dot(const LOp &op, bool unitary, const LOp &dot) {
+    const uint32_t ab = (1u << dot.sa) | (1u << dot.sb);
+    return !(op.smask & ab) || (unitary && (op.smask & ab) == ab);
+}
+
 // Two ops must keep their order when a bit they share is acted on
-// non-diagonally by one of them; read-only dots commute with each other.
-bool conflicts(const LOp &a, const LOp &b) {
+// non-diagonally by one of them, or when one is a dot that the other does not
+// leave as it is; read-only dots commute with each other.
+bool conflicts(const LOp &a, bool ua, const LOp &b, bool ub) {
     if (a.is_dot() && b.is_dot()) return false;
+    if (a.is_dot() && !passes_dot(b, ub, a)) return true;
+    if (b.is_dot() && !passes_dot(a, ua, b)) return true;
     const uint64_t na = a.nmask(), da = a.dmask() & ~na, nb = b.nmask(), db = b.dmask() & ~nb;
     return ((na & (nb | db)) | (da & nb)) != 0;
 }
@@ -624,14 +647,14 @@ bool reg_capable(const LOp &o) {
 // constraints between ops. Register bits of a stage are padded with the
 // previous stage's bits so that unchanged mappings need no transpose.
 template <typename LocalF>
-std::vector<StagePlan> plan_stages(const std::vector<LOp> &ops, const std::vector<int> &sel, LocalF local, int rb,
-                                   int kt) {
+std::vector<StagePlan> plan_stages(const std::vector<LOp> &ops, const std::vector<char> &unitary,
+                                   const std::vector<int> &sel, LocalF local, int rb, int kt) {
     const int m = static_cast<int>(sel.size());
     std::vector<std::vector<int>> succ(m);
     std::vector<int> indeg(m, 0);
     for (int j = 0; j < m; ++j)
         for (int i = 0; i < j; ++i)
-            if (conflicts(ops[sel[i]], ops[sel[j]])) {
+            if (conflicts(ops[sel[i]], unitary[sel[i]], ops[sel[j]], unitary[sel[j]])) {
                 succ[i].push_back(j);
                 ++indeg[j];
             }
@@ -1294,6 +1317,11 @@ std::vector<PassPlan> plan_passes(const std::vector<LOp> &ops, const PlanConfig 
         std::vector<int> D, RN, RD;
     };
     std::vector<BitDeps> bd(static_cast<size_t>(n));
+    // ops that a dot may not change places with on any bits, and the dots so far
+    const bool has_dots = std::any_of(ops.begin(), ops.end(), [](const LOp &o) { return o.is_dot(); });
+    const uint32_t all_states = (1u << cfg.ns) - 1u;
+    std::vector<char> unitary(N, 0);
+    std::vector<int> barriers, dots_seen;
     for (int j = 0; j < N; ++j) {
         nm[j] = ops[j].nmask();
         dm[j] = ops[j].dmask() & ~nm[j];
@@ -1337,9 +1365,20 @@ std::vector<PassPlan> plan_passes(const std::vector<LOp> &ops, const PlanConfig 
                 }
             }
         }
+        if (!has_dots) continue;
+        if (dot) {
+            for (int i : barriers)
+                if (!passes_dot(ops[i], unitary[i], ops[j])) dep(i);
+            dots_seen.push_back(j);
+        } else {
+            unitary[j] = ops[j].is_unitary(cfg.unitary_tol());
+            if (unitary[j] && (ops[j].smask & all_states) == all_states) continue;
+            for (int i : dots_seen)
+                if (!passes_dot(ops[j], unitary[j], ops[i])) dep(i);
+            barriers.push_back(j);
+        }
     }
 
-    const bool has_dots = std::any_of(ops.begin(), ops.end(), [](const LOp &o) { return o.is_dot(); });
     std::set<int> ready;
     for (int j = 0; j < N; ++j)
         if (indeg[j] == 0) ready.insert(j);
@@ -1492,7 +1531,7 @@ std::vector<PassPlan> plan_passes(const std::vector<LOp> &ops, const PlanConfig 
         std::vector<int> order = sel;
         std::vector<StagePlan> stages;
         if (p.reg) {
-            stages = plan_stages(ops, sel, local, cfg.reg_rb, kt);
+            stages = plan_stages(ops, unitary, sel, local, cfg.reg_rb, kt);
             order.clear();
             for (const auto &st : stages) order.insert(order.end(), st.ops.begin(), st.ops.end());
         }
@@ -1526,7 +1565,7 @@ std::vector<PassPlan> plan_passes(const std::vector<LOp> &ops, const PlanConfig 
             t.kind = o.kind;
             t.flags = o.flags;
             if (!o.is_dot() && o.is_swap()) t.flags |= TF_SWAP;
-            if (has_dots) t.flags |= o.is_dot() ? o.dot_class() : !cfg.keep_grouping && o.is_unitary() ? TF_UNITARY : 0u;
+            if (has_dots) t.flags |= o.is_dot() ? o.dot_class() : !cfg.keep_grouping && unitary[idx] ? TF_UNITARY : 0u;
             t.k = static_cast<uint32_t>(o.k);
             t.smask = o.smask;
             t.sa = o.sa;
@@ -1598,7 +1637,7 @@ std::string plan_structure_key(const std::vector<LOp> &ops, const PlanConfig &cf
             else if (o.k == 1 && o.coef.size() == 2 && o.coef[0] == mone && o.coef[1] == one) vflags = 2;
             else if (o.k == 0 && o.coef.size() == 1 && o.coef[0] == mone) vflags = 3;
         }
-        if (has_dots) vflags |= o.is_dot() ? o.dot_class() : o.is_unitary() ? TF_UNITARY : 0u;
+        if (has_dots) vflags |= o.is_dot() ? o.dot_class() : o.is_unitary(cfg.unitary_tol()) ? TF_UNITARY : 0u;
         // fields that are zero for most ops are written only where they are
         // not, behind a byte that says which
         const uint64_t m[8] = {o.cmask, o.cval, o.xmask, o.yzmask, o.pmask, o.pc_dim, static_cast<uint64_t>(o.ny),

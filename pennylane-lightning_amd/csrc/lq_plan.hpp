@@ -12,6 +12,13 @@
 
 namespace lqamd {
 
+// Dense operators on up to this many bits are tested for being unitary in
+// programs with dots: 5 us of host time on four bits, 33 on five, 245 on six,
+// each time the program is planned, for a dot that may be taken before the
+// operator instead of after it, at most one read of the state (50 us at 23
+// qubits). Wider ones count as not unitary.
+constexpr int kMaxUnitaryTest = 4;
+
 // An op on physical bits (bit b = wire n-1-b), before tiling.
 struct LOp {
     uint32_t kind = TOP_DIAG;
@@ -39,8 +46,9 @@ struct LOp {
     bool is_swap() const;
     // TF_DOT_X / TF_DOT_Y / TF_DOT_Z of a dot's operator, or 0
     uint32_t dot_class() const;
-    // U^dagger U = 1 (of the operator on its targets) to 1e-12
-    bool is_unitary() const;
+    // U^dagger U = 1 (of the operator on its targets) to tol; false also for
+    // dense operators on more than kMaxUnitaryTest bits
+    bool is_unitary(double tol) const;
 };
 
 inline int phys_bit(int n, uint32_t wire) { return n - 1 - static_cast<int>(wire); }
@@ -150,6 +158,11 @@ struct PlanConfig {
     // every amplitude by rounding, and expectation values, which come back in
     // double precision, by some 1e-7 of their size.
     bool keep_grouping = false;
+    // What counts as unitary for an op that a dot may change places with: the
+    // entries' rounding moves U^dagger U by two units of their precision (1.2e-7
+    // for a matrix that came in single precision, complex64 states), with room
+    // for a few products; past it a dot would be off by more than its rounding.
+    double unitary_tol() const { return keep_grouping ? 1e-6 : 1e-12; }
     // choose each pass's tile bits by lookahead (the bits that let the most
     // work run) instead of taking the first ready op's bits
     bool lookahead = false;
