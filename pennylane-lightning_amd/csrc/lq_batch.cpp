@@ -136,8 +136,12 @@ namespace {
 constexpr size_t kRunnerInBytes = 64u << 20;
 constexpr size_t kRunnerOutBytes = 1u << 20;
 constexpr size_t kSectionAlign = 256; // each of the 5 sections starts 256-byte aligned
-} // namespace
 
+// A stream with a hardware queue of its own where the device grants one (null
+// on failure): a CU-masked stream (every CU enabled) gets a new queue instead
+// of sharing one with other streams once the process's queue pool is full,
+// where it would wait behind their kernels. It is ordered with the null stream
+// (its creation takes no flags).
 hipStream_t own_queue_stream() {
     int dev = 0, cus = 0;
     const char *oq = std::getenv("LQ_BATCH_OWN_QUEUE");
@@ -151,6 +155,7 @@ hipStream_t own_queue_stream() {
     if (hipExtStreamCreateWithCUMask(&s, static_cast<uint32_t>(mask.size()), mask.data()) != hipSuccess) return nullptr;
     return s;
 }
+} // namespace
 
 BatchRunner::BatchRunner() {
     const char *ku = std::getenv("LQ_BATCH_KERNEL_UPLOAD");

@@ -80,12 +80,6 @@ struct BatchProgram {
 bool build_batch_program(int n, int dtype, const OpsList &ops, const Obs &ham, const std::vector<uint64_t> &tp,
                          BatchProgram *out, std::string *why);
 
-// A stream with a hardware queue of its own where the device grants one (null
-// on failure): a CU-masked stream (every CU enabled) gets a new queue instead
-// of sharing one of the process's few with other streams, where it would wait
-// behind their kernels.
-hipStream_t own_queue_stream();
-
 // Device buffers + stream for packed launches (one per concurrent launch).
 class BatchRunner {
   public:

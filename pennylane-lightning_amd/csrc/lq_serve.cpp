@@ -259,16 +259,20 @@ void Server::run_engine(StateVector &sv, Req &r) {
 void Server::large_loop(bool lane) {
     (void)hipSetDevice(device_);
     // the worker's own stream: the pooled states it takes run on it, so the
-    // server's streams are its workers and packed runners only, each with a
-    // hardware queue of its own (states keep their own streams while idle).
-    // Ordinary streams share the process's hardware queues (four, or
-    // GPU_MAX_HW_QUEUES), and kernels of one queue run one after the other: ten
-    // workers' passes of four to sixteen workgroups took 18.9 ms for 64
-    // requests of 10 to 15 qubits on four queues, 14.8 ms on their own.
-    // (If no stream can be created, requests run on the states' own streams:
+    // server's streams are its workers and packed runners only (states keep
+    // their own streams while idle). Non-blocking: work that the process puts
+    // on the null stream (torch's default) must not wait for the workers'
+    // kernels, nor they for it. A CU-masked stream would give a worker a
+    // hardware queue of its own where the process has fewer than it has
+    // streams (64 requests of 10 to 15 qubits on four queues: 14.8 ms in place
+    // of 18.9), but its creation takes no flags and it is ordered with the null
+    // stream: an addition on torch's default stream waited 57 ms for 58 ms of
+    // such a stream's kernels, 7 ms (the kernel then running) beside a
+    // non-blocking one.
+    // (If it cannot be created, requests run on the states' own streams:
     // nothing may throw out of a worker thread.)
-    hipStream_t ws = own_queue_stream();
-    if (!ws && hipStreamCreateWithFlags(&ws, hipStreamNonBlocking) != hipSuccess) ws = nullptr;
+    hipStream_t ws = nullptr;
+    if (hipStreamCreateWithFlags(&ws, hipStreamNonBlocking) != hipSuccess) ws = nullptr;
     struct StreamGuard {
         hipStream_t s;
         ~StreamGuard() {
