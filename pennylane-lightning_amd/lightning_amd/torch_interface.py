@@ -62,7 +62,18 @@ def num_params(ops) -> int:
     return sum(len(op.params) for op in ops)
 
 
-_ONE_WIRE = frozenset(("PauliX", "PauliY", "PauliZ", "Hadamard", "Identity"))
+# (not the identity: a batch takes it as 1, an observable's mean is the state's norm)
+_ONE_WIRE = frozenset(("PauliX", "PauliY", "PauliZ", "Hadamard"))
+
+
+def _one_wire_batch(observables, n):
+    """Names and wires of several named observables that one program can
+    evaluate (wires in range; others raise where they are evaluated alone), or
+    None."""
+    if len(observables) < 2 or not all(o[0] == "N" and o[1] in _ONE_WIRE for o in observables):
+        return None
+    wires = [int(o[2]) for o in observables]
+    return ([o[1] for o in observables], wires) if all(0 <= w < n for w in wires) else None
 
 
 class _CircuitExpvals(torch.autograd.Function):
@@ -73,10 +84,11 @@ class _CircuitExpvals(torch.autograd.Function):
         sv = (L.StateVectorC128 if bits == 128 else L.StateVectorC64)(n)
         apply_circuit(sv, bound)
         m = (L.MeasurementsC128 if bits == 128 else L.MeasurementsC64)(sv)
-        if bits == 128 and len(observables) > 1 and all(o[0] == "N" and o[1] in _ONE_WIRE for o in observables):
-            # one program for the circuit and all of them (in single precision
-            # another set of dots means other passes and another rounding)
-            ev = m.expval_named_batch([o[1] for o in observables], [o[2] for o in observables])
+        # one program for the circuit and all of them (in single precision
+        # another set of dots means other passes and another rounding)
+        batch = _one_wire_batch(observables, n) if bits == 128 else None
+        if batch:
+            ev = m.expval_named_batch(*batch)
         else:
             ev = np.array([m.expval(observable(o, bits)) for o in observables], dtype=np.float64)
         ctx.sv, ctx.bound, ctx.observables, ctx.bits = sv, bound, observables, bits
