@@ -146,10 +146,12 @@ def check(rc: int) -> None:
 
 
 def u32(xs):
+    if not isinstance(xs, (list, tuple)):
+        xs = list(xs)
     try:
         a = array("I", xs)
-    except (TypeError, ValueError):  # floats, nested lists, tensors
-        a = array("I", np.ascontiguousarray(np.asarray(list(xs), dtype=np.uint32).reshape(-1)).tolist())
+    except TypeError:  # floats, nested lists, tensors
+        a = array("I", np.ascontiguousarray(np.asarray(xs, dtype=np.uint32).reshape(-1)).tolist())
     n = len(a)
     if n == 0:
         a.append(0)
