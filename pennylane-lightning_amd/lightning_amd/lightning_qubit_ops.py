@@ -361,11 +361,11 @@ class _StateVectorBase:
         if n == 0:
             return
         blob = b"\0".join(map(_NAME_BYTES.__getitem__, ops)) + b"\0"
-        woff, wflat = _flatten("I", wires)
+        woff, wflat = _flatten("I", wires, iterators=False)
         inv = _flags(inverses)
         poff = pfl = None
         if params is not None:
-            poff, pfl = _flatten("d", params)
+            poff, pfl = _flatten("d", params, iterators=False)
         check(lib.lq_sv_apply_operations(self._h, n, blob, _addr(woff, C.c_uint32), _addr(wflat, C.c_uint32),
                                          _addr(inv, C.c_uint8), _addr(poff, C.c_uint32), _addr(pfl, C.c_double)))
 
@@ -454,12 +454,14 @@ def _name_bytes(name: str) -> bytes:
     return _NAME_BYTES[name]
 
 
-def _flatten(code, lists):
+def _flatten(code, lists, iterators=True):
     """Offsets (uint32, one more than lists) and the concatenated values of
-    type ``code`` (array module)."""
+    type ``code`` (array module); ``iterators``: entries may have no length."""
     try:
         off = array("I", accumulate(map(len, lists), initial=0))
-    except TypeError:  # iterators
+    except TypeError:
+        if not iterators:
+            raise
         lists = [list(v) for v in lists]
         off = array("I", accumulate(map(len, lists), initial=0))
     try:
@@ -471,6 +473,8 @@ def _flatten(code, lists):
 
 def _first(lists, n):
     """The first n entries; fewer are an error, as indexing them would be."""
+    if not hasattr(lists, "__len__"):
+        lists = list(lists)
     if len(lists) < n:
         raise IndexError("list index out of range")
     return lists if len(lists) == n else lists[:n]

@@ -8,9 +8,24 @@ from lightning_amd import workloads as W
 from lightning_amd._capi import u32
 
 
+@pytest.mark.parametrize("rows", [lambda v: (x for x in v), lambda v: map(tuple, v), lambda v: [iter(x) for x in v]])
+def test_ops_struct_from_iterators(rows):
+    ops = L.OpsStructC128(["RX", "CRY"], rows([[0.1], [0.2]]), rows([[0], [1]]), iter([False, True]), iter([[], []]),
+                          rows([[], [2]]), rows([[], [True]]))
+    assert ops.params == [[0.1], [0.2]] and ops.wires == [[0], [1]] and ops.inverses == [False, True]
+    assert ops.ctrl_wires == [[], [2]] and ops.ctrl_values == [[], [True]]
+
+
 @pytest.mark.parametrize("values,expected", [(lambda: (float(i) for i in (1, 2, 3)), [1, 2, 3]),
                                              (lambda: (i for i in ()), []), (lambda: b"\0\1\2\3", [0, 1, 2, 3]),
                                              (lambda: bytearray(b"\0\1\2\3"), [0, 1, 2, 3]), (lambda: {3: 1}, [3])])
 def test_wire_iterators_and_bytes(values, expected):
     a, p, n = u32(values())
     assert [p[i] for i in range(n)] == expected
+
+
+def test_gate_lists_without_length_are_refused():
+    sv = object.__new__(L.StateVectorC128)
+    for wires, params in (([iter([0])], [[0.1]]), ([[0]], [iter([0.1])])):
+        with pytest.raises(TypeError):
+            sv.applyOperations(["RX"], wires, [False], params)
