@@ -28,6 +28,7 @@ import ctypes as C
 import sys
 import types
 from array import array
+from functools import cached_property
 from itertools import accumulate, chain
 from typing import Sequence
 
@@ -804,8 +805,8 @@ class OpsStruct:
         self.inverses = list(map(bool, ops_inverses))
         self.matrices = [_NO_MATRIX if m is None or not len(m) else np.asarray(m, dtype=np.complex128).reshape(-1)
                          for m in _first(ops_matrices, n)]
-        # flat copies, as the engine takes them; ``params``, ``wires`` and the
-        # controls are read back from them
+        # flat copies, as the engine takes them; the lists ``params``, ``wires``
+        # and the controls are made from them when first asked for
         self._params = poff, params = _flatten("d", _first(ops_params, n))
         self._wires = woff, wires = _flatten("I", _first(ops_wires, n))
         self._ctrls = coff, ctrls = _flatten("I", _first(ops_controlled_wires, n))
@@ -831,19 +832,19 @@ class OpsStruct:
     def _lists(off, values):
         return [list(values[off[i]:off[i + 1]]) for i in range(len(off) - 1)]
 
-    @property
+    @cached_property
     def params(self):
         return self._lists(*self._params)
 
-    @property
+    @cached_property
     def wires(self):
         return self._lists(*self._wires)
 
-    @property
+    @cached_property
     def ctrl_wires(self):
         return self._lists(*self._ctrls)
 
-    @property
+    @cached_property
     def ctrl_values(self):
         return [[bool(v) for v in vs] for vs in self._lists(self._cvals_off, self._cvals)]
 

@@ -16,6 +16,14 @@ def test_ops_struct_from_iterators(rows):
     assert ops.ctrl_wires == [[], [2]] and ops.ctrl_values == [[], [True]]
 
 
+def test_ops_struct_lists_are_attributes():
+    ops = L.OpsStructC128(["RX"], [[0.1]], [[0]], [False], [[]])
+    ops.params = [[5.0]]
+    ops.wires.append([3])
+    assert ops.params == [[5.0]] and ops.wires == [[0], [3]]
+    assert ops.ctrl_wires is ops.ctrl_wires and ops.ctrl_values is ops.ctrl_values
+
+
 @pytest.mark.parametrize("values,expected", [(lambda: (float(i) for i in (1, 2, 3)), [1, 2, 3]),
                                              (lambda: (i for i in ()), []), (lambda: b"\0\1\2\3", [0, 1, 2, 3]),
                                              (lambda: bytearray(b"\0\1\2\3"), [0, 1, 2, 3]), (lambda: {3: 1}, [3])])
