@@ -50,6 +50,8 @@ def bind(ops, values):
     it = iter(np.asarray(values, dtype=np.float64).tolist())
 
     def bound(op):
+        if type(op) is not CircuitOp:
+            return CircuitOp(op.name, op.wires, [next(it) for _ in op.params], op.inverse, op.matrix, op.ctrls, op.cvals)
         out = object.__new__(CircuitOp)
         out.__dict__.update(op.__dict__)
         out.params = [next(it) for _ in op.params]

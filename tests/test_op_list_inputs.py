@@ -37,3 +37,17 @@ def test_gate_lists_without_length_are_refused():
     for wires, params in (([iter([0])], [[0.1]]), ([[0]], [iter([0.1])])):
         with pytest.raises(TypeError):
             sv.applyOperations(["RX"], wires, [False], params)
+
+
+def test_bind_takes_any_op():
+    T = pytest.importorskip("lightning_amd.torch_interface")
+
+    class Op:
+        name, wires, params, inverse, matrix, ctrls, cvals = "RX", [0], [0.1], False, None, [], []
+
+    class Derived(W.CircuitOp):
+        pass
+
+    expected = W.CircuitOp("RX", [0], [0.7])
+    for op in (Op(), Derived("RX", [0], [0.1]), W.CircuitOp("RX", [0], [0.1])):
+        assert T.bind([op], [0.7]) == [expected]
