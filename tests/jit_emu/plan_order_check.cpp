@@ -8,11 +8,14 @@
 //   cz:         the same with runs of CZ in either order of its wires, CCZ and phases
 //   nonunitary: operators that are not unitary among the gates (one to three wires, with
 //               and without controls, zeroing generators), dots after and between them
+//   long:       8000 gates in one pass, on a few wires and on all; planning takes at most
+//               24 times as long as for 1000 gates (8 times the ops; 64 if pair by pair)
 //   partial:    two and three states, gates on some of them only, dots between them
 // Each program is planned on 12 to 14 qubits, with one to three states, plain and with
 // split rotations, and with the grouping of either precision. Exit status 0 when nothing
 // is off by more than 1e-10 of the states' norms: a split gate is exact to 1e-13 of its
 // amplitudes, and no program has more than 200 gates.
+#include <chrono>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -288,9 +291,67 @@ static void not_unitary(Builder &b, uint32_t sm) {
     }
 }
 
+// Gates of a program for the family "long".
+static std::vector<LOp> long_program(int n, int wires, int count) {
+    Builder b(n, 1, 41);
+    b.n = wires; // gates on the first wires, lowered for n qubits below
+    std::vector<LOp> prog;
+    const GateId one[] = {GateId::RX, GateId::RZ, GateId::Rot};
+    while (static_cast<int>(prog.size()) < count) {
+        const bool two = b.below(2) != 0;
+        const std::vector<uint32_t> w = b.wires(two ? 2 : 1);
+        const double p[3] = {b.angle(), b.angle(), b.angle()};
+        LOp op = lower_gate(n, two ? GateId::CNOT : one[b.below(3)], w.data(), static_cast<int>(w.size()), nullptr, nullptr,
+                            0, false, p);
+        if (!try_merge_1q(prog, op)) prog.push_back(std::move(op));
+    }
+    return prog;
+}
+
+static int long_passes() {
+    int wrong = 0;
+    for (int wires : {4, 12}) {
+        PlanConfig cfg;
+        cfg.n = 12;
+        cfg.kt_max = 12;
+        cfg.reg_rb = 4;
+        cfg.max_dots = 32;
+        cfg.budget = 1e9;
+        double best[2] = {1e9, 1e9};
+        std::vector<PassPlan> plan;
+        for (int k = 0; k < 2; ++k) {
+            const std::vector<LOp> prog = long_program(12, wires, k ? 8000 : 1000);
+            for (int r = 0; r < 5; ++r) {
+                const auto t = std::chrono::steady_clock::now();
+                plan = plan_passes(prog, cfg);
+                best[k] = std::min(best[k], std::chrono::duration<double>(std::chrono::steady_clock::now() - t).count());
+            }
+            std::vector<State> ref(1, State(1ull << 12)), got;
+            ref[0][5] = 1.0;
+            got = ref;
+            std::vector<cd> none;
+            program_order(ref, prog, none);
+            planned_order(got, 12, plan, none);
+            double err = 0.0;
+            for (size_t i = 0; i < ref[0].size(); ++i) err = std::max(err, std::abs(ref[0][i] - got[0][i]));
+            const bool ok = err <= 1e-10 && plan.size() == 1;
+            std::printf("%d wires, %zu gates: %zu passes, off by %.1e, planned in %.2f ms\n", wires, prog.size(), plan.size(),
+                        err, best[k] * 1e3);
+            wrong += !ok;
+        }
+        if (!(best[1] <= 24.0 * best[0])) {
+            std::printf("%d wires: planning is not linear in the gates\n", wires);
+            ++wrong;
+        }
+    }
+    std::printf("long: 4 plans, %d wrong\n", wrong);
+    return wrong ? 1 : 0;
+}
+
 int main(int argc, char **argv) {
     const std::string family = argc > 1 ? argv[1] : "words";
     const unsigned seeds = argc > 2 ? static_cast<unsigned>(std::atoi(argv[2])) : 100;
+    if (family == "long") return long_passes();
     int wrong = 0, plans = 0;
     double worst = 0.0;
     for (unsigned seed = 0; seed < seeds; ++seed) {

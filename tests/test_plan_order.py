@@ -29,7 +29,7 @@ def checker(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("family,seeds", [("words", 500), ("cz", 200), ("nonunitary", 200), ("partial", 200)])
+@pytest.mark.parametrize("family,seeds", [("words", 500), ("cz", 200), ("nonunitary", 200), ("partial", 200), ("long", 1)])
 def test_plans_keep_the_order_of_their_ops(checker, family, seeds):
     r = subprocess.run([checker, family, str(seeds)], capture_output=True, text=True, timeout=600)
     assert r.returncode == 0, r.stdout[-3000:] + r.stderr[-2000:]
