@@ -402,7 +402,12 @@ struct BitList {
 // histogram and no atomics, so any number of wires takes the same route and
 // the sums do not depend on scheduling. 26 qubits complex128, 14 scattered
 // wires: 3.19 ms (one thread per output gathering 2^12 scattered amplitudes)
-// -> 0.16 ms, the read of 1 GiB at 6.5 TB/s.
+// -> 0.16 ms, the read of 1 GiB at 6.5 TB/s. Where nearly all high bits are
+// measured an item is one load a thread, so what an item costs besides counts:
+// its bits are put in place by one ballot each (lane L answers for bit L of the
+// index, then for bit L of the output), not by a loop over the bits, and a
+// workgroup takes many items (24 qubits, the 16 high wires: 227 -> 101 us
+// for the call; by gathers 174).
 template <typename T>
 __global__ __launch_bounds__(kBlock) void probs_kernel(const typename VecT<T>::type *__restrict__ a, int lb,
                                                       uint32_t wl, uint64_t wh, uint64_t sm, uint64_t rm,
@@ -412,17 +417,21 @@ __global__ __launch_bounds__(kBlock) void probs_kernel(const typename VecT<T>::t
     const uint32_t tid = threadIdx.x;
     const uint32_t rest = ((1u << lb) - 1u) & ~wl; // unmeasured low bits, summed across threads
     const uint64_t count = 1ull << __popcll(rm);
+    const uint32_t lane = tid & 63u;
+    // the item's bit that stands at state bit `lane`: measured high bits
+    // first, then the split bits
+    const uint64_t below = (1ull << lane) - 1ull;
+    const int mine = (wh >> lane) & 1ull   ? __popcll(wh & below)
+                     : (sm >> lane) & 1ull ? __popcll(wh) + __popcll(sm & below)
+                                           : -1;
+    // the high state bit that output bit `lane` stands for
+    const int from = lane < static_cast<uint32_t>(nw) && bits.b[lane] >= lb ? bits.b[lane] : -1;
     uint64_t olow = 0; // this thread's part of the output index
     for (int j = 0; j < nw; ++j)
-        if (bits.b[j] < lb) olow |= static_cast<uint64_t>((tid >> bits.b[j]) & 1u) << (nw - 1 - j);
+        if (bits.b[j] < lb) olow |= static_cast<uint64_t>((tid >> bits.b[j]) & 1u) << j;
     for (uint64_t item = blockIdx.x; item < items; item += gridDim.x) {
-        // deposit the item number: measured high bits first, then the split bits
-        uint64_t base = 0, x = item;
-        for (uint64_t m = wh; m; m &= m - 1, x >>= 1)
-            if (x & 1ull) base |= m & (~m + 1);
-        const uint64_t row = x;
-        for (uint64_t m = sm; m; m &= m - 1, x >>= 1)
-            if (x & 1ull) base |= m & (~m + 1);
+        const uint64_t base = __ballot(mine >= 0 && ((item >> (mine & 63)) & 1ull));
+        const uint64_t row = item >> __popcll(wh);
         double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
         if (tid < (1u << lb)) {
             const typename VecT<T>::type *p = a + (base | tid);
@@ -457,12 +466,8 @@ __global__ __launch_bounds__(kBlock) void probs_kernel(const typename VecT<T>::t
             }
             __syncthreads(); // red is reused by the next item
         }
-        if (tid < (1u << lb) && (tid & rest) == 0) {
-            uint64_t o = olow;
-            for (int j = 0; j < nw; ++j)
-                if (bits.b[j] >= lb) o |= ((base >> bits.b[j]) & 1ull) << (nw - 1 - j);
-            out[(row << nw) + o] = s;
-        }
+        const uint64_t ohigh = __ballot(from >= 0 && ((base >> (from & 63)) & 1ull));
+        if (tid < (1u << lb) && (tid & rest) == 0) out[(row << nw) + (olow | ohigh)] = s;
     }
 }
 
@@ -746,6 +751,11 @@ template void launch_sparse_rows<double>(const void *, void *, const int64_t *, 
 template void launch_sparse_rows<float>(const void *, void *, const int64_t *, const int64_t *, const void *, uint64_t,
                                         int, double2 *, uint32_t, hipStream_t);
 
+// Workgroups of a marginal: two rounds of the eight a CU holds; each then takes
+// several items (22 and 24 qubits, the 16 high wires: 61 and 101 us with 2048,
+// 63 and 101 with 4096, 75 and 104 with 16384).
+constexpr uint64_t kProbsBlocks = 4096;
+
 // High bits of a marginal: measured (wh) and not (rest), and how many of the
 // unmeasured ones (the highest) are split over workgroups. Eight workgroups
 // for each of the 256 CUs fill the chip, but an item keeps at least four
@@ -782,9 +792,11 @@ template <typename T> void launch_probs(const void *a, int n, const int *bits, i
     for (int j = 0; j < nw; ++j)
         if (bits[j] < lb) wl |= 1u << bits[j];
     const uint64_t items = 1ull << (__builtin_popcountll(wh) + split);
-    const uint32_t grid = static_cast<uint32_t>(items < (1u << 20) ? items : (1u << 20));
+    int from[64] = {}; // state bit of each output bit
+    for (int j = 0; j < nw; ++j) from[nw - 1 - j] = bits[j];
+    const uint32_t grid = static_cast<uint32_t>(std::min<uint64_t>(items, kProbsBlocks));
     hipLaunchKernelGGL(probs_kernel<T>, dim3(grid), dim3(kBlock), 0, s, static_cast<const V *>(a), lb, wl, wh, sm, rm,
-                       items, to_bitlist(bits, nw), nw, out);
+                       items, to_bitlist(from, nw), nw, out);
 }
 template void launch_probs<double>(const void *, int, const int *, int, double *, hipStream_t);
 template void launch_probs<float>(const void *, int, const int *, int, double *, hipStream_t);
