@@ -108,11 +108,19 @@ bool LOp::is_unitary(double tol) const {
     }
     const size_t d = static_cast<size_t>(1) << k;
     if (k > kMaxUnitaryTest || coef.size() != d * d) return false;
+    // rows against rows, over the columns where neither is zero (the rows of a
+    // gate that leaves most basis states alone have one entry each)
+    uint32_t filled[1u << kMaxUnitaryTest];
+    for (size_t a = 0; a < d; ++a) {
+        filled[a] = 0;
+        for (size_t c = 0; c < d; ++c)
+            if (coef[a * d + c] != cd(0.0)) filled[a] |= 1u << c; // NaN too
+    }
     for (size_t a = 0; a < d; ++a)
         for (size_t b = a; b < d; ++b) {
             double re = a == b ? -1.0 : 0.0, im = 0.0;
-            for (size_t r = 0; r < d; ++r) {
-                const cd u = coef[r * d + a], v = coef[r * d + b];
+            for (uint32_t m = filled[a] & filled[b]; m; m &= m - 1) {
+                const cd u = coef[a * d + static_cast<size_t>(__builtin_ctz(m))], v = coef[b * d + static_cast<size_t>(__builtin_ctz(m))];
                 re += u.real() * v.real() + u.imag() * v.imag();
                 im += u.real() * v.imag() - u.imag() * v.real();
             }

@@ -13,7 +13,7 @@
 namespace lqamd {
 
 // Dense operators on up to this many bits are tested for being unitary in
-// programs with dots: 5 us of host time on four bits, 33 on five, 245 on six,
+// programs with dots: up to 4 us of host time on four bits, 33 on five, 245 on six,
 // each time the program is planned, for a dot that may be taken before the
 // operator instead of after it, at most one read of the state (50 us at 23
 // qubits). Wider ones count as not unitary.
