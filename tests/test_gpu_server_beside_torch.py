@@ -24,6 +24,8 @@ def test_default_stream_runs_beside_engine_workers():
     words = [[("PauliZ", w), ("PauliX", (w + 1) % n)] for w in range(n)]
     srv = S.Server(bits=128, batched=True, large_workers=2)
     reqs = [S.Request(n, 4, ops, [1.0] * n, words, 128) for _ in range(12)]
+    for r in reqs:
+        r.handles()  # op lists are made before the time starts
     srv.run(reqs[0])
     L.jit_wait()
     srv.run(reqs[0])
