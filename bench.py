@@ -490,7 +490,7 @@ def run_mfma5(args):
     """Matrix cores for fused dense blocks, complex64: one Haar-random 32x32
     unitary on wires 25..29 of a 30-qubit complex64 state (the five lowest
     index bits), applied (a) as a 64x64 real GEMM per 32-amplitude group on
-    the MFMA units, (b) as a dense tile op in the engine's default path, and
+    the MFMA units, (b) in the planner's dense pass (as for any five wires), and
     (c) the gates such a block fuses in the hardware-efficient ansatz (one
     layer on those wires: 5 Rot + 4 CZ) through the engine's specialised
     passes. Times per application (stream-synchronised), HBM rate over

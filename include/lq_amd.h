@@ -336,7 +336,8 @@ int lq_set_split_fallback(int mode, int *previous);
  * lowest index bits (wires n-5 .. n-1 in any order) without controls:
  * with on != 0, applyMatrix of such an operator runs as one 64x64 real
  * GEMM per 32-amplitude group on the MFMA units (v_mfma_f32_16x16x4_f32)
- * instead of as a fused tile op; default on (LQ_MFMA_DENSE5). Replaces the
+ * at once, instead of in a dense pass among the queued gates; default on
+ * (LQ_MFMA_DENSE5). Replaces the
  * dense k-qubit kernel for that case (lq/gates/cpu_kernels/
  * GateImplementationsLM.hpp:454-498, applyNQubitOp). */
 int lq_set_mfma_dense5(int on, int *previous);

@@ -145,9 +145,6 @@ LOp identity_dot(uint32_t sa, uint32_t sb, int slot, uint32_t part = 0) {
     return make_dot(op, sa, sb, slot, part);
 }
 
-// Pauli word as the cheapest op form for a dot: a parity op for Z-only
-// words, a dense 2x2 / 4x4 (or diagonal) op for words on one or two qubits,
-// the general Pauli-string op otherwise.
 // Kernel terms of a Pauli sum, in order of x (launch_pauli_sum). For an
 // expectation only the real part of a word's coefficient counts, and words
 // with x != 0 count twice for half of the index pairs.
@@ -181,6 +178,9 @@ std::vector<uint32_t> pauli_groups(const std::vector<PauliTerm> &terms, int n, i
     return ends;
 }
 
+// Pauli word as the cheapest op form for a dot: a parity op for Z-only
+// words, a dense 2x2 / 4x4 (or diagonal) op for words on one or two qubits,
+// the general Pauli-string op otherwise.
 LOp pauli_dot_op(int n, const PauliWord &w) {
     (void)n;
     const uint64_t sup = w.x | w.yz;

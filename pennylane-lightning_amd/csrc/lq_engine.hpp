@@ -99,7 +99,7 @@ struct OpsList {
 };
 
 // Dense operators on more targets than this run out of place through a
-// global-memory kernel instead of as tile ops.
+// global-memory kernel instead of in the planner's passes.
 constexpr int kMaxFusedTargets = 10;
 // From this many qubits, specialised programs are planned under several
 // pass budgets and the plan with the fewest passes is kept.
@@ -120,10 +120,11 @@ struct EngineTuning {
     // (written through lq_set_split_fallback while other threads plan)
     std::atomic<int> split_fallback{1};
     // complex64 dense operators on exactly the five lowest index bits (no
-    // controls) run as a 64x64 real GEMM on the matrix cores instead of as a
-    // tile op (lq_set_mfma_dense5 / LQ_MFMA_DENSE5)
-    // (measured on a 30-qubit complex64 state: 3.4 ms per operator against
-    // 167 ms as a tile op; on by default)
+    // controls) run at once as a 64x64 real GEMM on the matrix cores instead
+    // of in a dense pass among the queued gates (lq_set_mfma_dense5 /
+    // LQ_MFMA_DENSE5; on by default)
+    // (per operator, 3.36 ms against 3.66 at 30 qubits and 0.84 against 0.86
+    // at 28; 228 us against 218 at 26, 29 against 18 at 20)
     std::atomic<int> mfma_dense5{1};
     // Leading one-qubit gates after a reset fold into the product state the
     // first pass forms, and for large states several pass budgets are planned

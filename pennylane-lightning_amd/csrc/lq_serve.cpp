@@ -264,9 +264,9 @@ void Server::large_loop(bool lane) {
     // on the null stream (torch's default) must not wait for the workers'
     // kernels, nor they for it. A CU-masked stream would give a worker a
     // hardware queue of its own where the process has fewer than it has
-    // streams (64 requests of 10 to 15 qubits on four queues: 14.8 ms in place
-    // of 18.9), but its creation takes no flags and it is ordered with the null
-    // stream: an addition on torch's default stream waited 57 ms for 58 ms of
+    // streams (64 requests of 10 to 15 qubits, four queues in the pool: 15.6 to
+    // 16.4 ms, in turn 15.9 to 16.5 without), but its creation takes no flags
+    // and it is ordered with the null stream: an addition on torch's default stream waited 57 ms for 58 ms of
     // such a stream's kernels, 7 ms (the kernel then running) beside a
     // non-blocking one.
     // (If it cannot be created, requests run on the states' own streams:
