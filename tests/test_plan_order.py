@@ -14,7 +14,7 @@ LIB = os.path.join(PKG, "lightning_amd", "_lib")
 
 
 @pytest.fixture(scope="module")
-def checker(tmp_path_factory):
+def compiled(tmp_path_factory):
     if not os.path.exists(os.path.join(LIB, "liblq_amd.so")):
         pytest.skip("liblq_amd.so not built")
     hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
@@ -30,7 +30,7 @@ def checker(tmp_path_factory):
 
 
 @pytest.mark.parametrize("family,seeds", [("words", 500), ("cz", 200), ("nonunitary", 200), ("partial", 200), ("long", 1)])
-def test_plans_keep_the_order_of_their_ops(checker, family, seeds):
-    r = subprocess.run([checker, family, str(seeds)], capture_output=True, text=True, timeout=600)
+def test_plans_keep_the_order_of_their_ops(compiled, family, seeds):
+    r = subprocess.run([compiled, family, str(seeds)], capture_output=True, text=True, timeout=600)
     assert r.returncode == 0, r.stdout[-3000:] + r.stderr[-2000:]
     assert f"{4 * seeds} plans, 0 wrong" in r.stdout
