@@ -16,6 +16,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 #include <queue>
 #include <set>
 
@@ -91,7 +92,7 @@ uint32_t LOp::dot_class() const {
     return 0;
 }
 
-bool LOp::is_unitary(double tol) const {
+bool LOp::is_unitary(double tol, int max_k) const {
     if (flags & TF_ZERO_UNCTRL) return false;
     switch (kind) {
     case TOP_DIAG:
@@ -107,23 +108,33 @@ bool LOp::is_unitary(double tol) const {
     default: return false;
     }
     const size_t d = static_cast<size_t>(1) << k;
-    if (k > kMaxUnitaryTest || coef.size() != d * d) return false;
-    // rows against rows, over the columns where neither is zero (the rows of a
-    // gate that leaves most basis states alone have one entry each)
-    uint32_t filled[1u << kMaxUnitaryTest];
+    if (k > max_k || k > 6 || coef.size() != d * d) return false;
+    // rows against rows; those without a column that both fill need no product
+    // (a gate that leaves most basis states alone has rows of one entry)
+    uint64_t filled[64];
     for (size_t a = 0; a < d; ++a) {
         filled[a] = 0;
         for (size_t c = 0; c < d; ++c)
-            if (coef[a * d + c] != cd(0.0)) filled[a] |= 1u << c; // NaN too
+            if (coef[a * d + c] != cd(0.0)) filled[a] |= 1ull << c; // NaN too
     }
+    typedef double v2 __attribute__((vector_size(16))); // (re, im)
+    auto load = [&](size_t i) {
+        v2 x;
+        std::memcpy(&x, &coef[i], sizeof(x));
+        return x;
+    };
     for (size_t a = 0; a < d; ++a)
         for (size_t b = a; b < d; ++b) {
-            double re = a == b ? -1.0 : 0.0, im = 0.0;
-            for (uint32_t m = filled[a] & filled[b]; m; m &= m - 1) {
-                const cd u = coef[a * d + static_cast<size_t>(__builtin_ctz(m))], v = coef[b * d + static_cast<size_t>(__builtin_ctz(m))];
-                re += u.real() * v.real() + u.imag() * v.imag();
-                im += u.real() * v.imag() - u.imag() * v.real();
-            }
+            if (!(filled[a] & filled[b]) && a != b) continue;
+            v2 p[2] = {}, q[2] = {}; // u v, and u times v with its parts exchanged
+            for (size_t c = 0; c < d; c += 2)
+                for (size_t j = 0; j < 2; ++j) {
+                    const v2 u = load(a * d + c + j), v = load(b * d + c + j);
+                    p[j] += u * v;
+                    q[j] += u * v2{v[1], v[0]};
+                }
+            const v2 ps = p[0] + p[1], qs = q[0] + q[1];
+            const double re = ps[0] + ps[1] - (a == b ? 1.0 : 0.0), im = qs[0] - qs[1];
             if (!(re * re + im * im <= tol * tol)) return false;
         }
     return true;
@@ -1418,7 +1429,7 @@ std::vector<PassPlan> plan_passes(const std::vector<LOp> &ops, const PlanConfig 
         cost_of[j] = ops[j].cost();
         if (cfg.lookahead && !cfg.keep_grouping && !ops[j].is_dot() && ops[j].is_swap()) cost_of[j] *= kSwapCost / (ops[j].k == 1 ? 1.0 : 2.5);
         LQ_ABORT_IF(((nm[j] | dm[j]) >> n) != 0, "operation acts on a wire outside the state");
-        if (has_dots && !ops[j].is_dot()) unitary[j] = ops[j].is_unitary(cfg.unitary_tol());
+        if (has_dots && !ops[j].is_dot()) unitary[j] = ops[j].is_unitary(cfg.unitary_tol(), cfg.max_unitary_test());
     }
     OpOrder whole = order_ops(ops, all, nm, dm, unitary, n, cfg.ns);
     std::vector<std::vector<int>> &succ = whole.succ;
@@ -1682,7 +1693,7 @@ std::string plan_structure_key(const std::vector<LOp> &ops, const PlanConfig &cf
             else if (o.k == 1 && o.coef.size() == 2 && o.coef[0] == mone && o.coef[1] == one) vflags = 2;
             else if (o.k == 0 && o.coef.size() == 1 && o.coef[0] == mone) vflags = 3;
         }
-        if (has_dots) vflags |= o.is_dot() ? o.dot_class() : o.is_unitary(cfg.unitary_tol()) ? TF_UNITARY : 0u;
+        if (has_dots) vflags |= o.is_dot() ? o.dot_class() : o.is_unitary(cfg.unitary_tol(), cfg.max_unitary_test()) ? TF_UNITARY : 0u;
         // fields that are zero for most ops are written only where they are
         // not, behind a byte that says which
         const uint64_t m[8] = {o.cmask, o.cval, o.xmask, o.yzmask, o.pmask, o.pc_dim, static_cast<uint64_t>(o.ny),

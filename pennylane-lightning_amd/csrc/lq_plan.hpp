@@ -12,13 +12,6 @@
 
 namespace lqamd {
 
-// Dense operators on up to this many bits are tested for being unitary in
-// programs with dots: up to 4 us of host time on four bits, 33 on five, 245 on six,
-// each time the program is planned, for a dot that may be taken before the
-// operator instead of after it, at most one read of the state (50 us at 23
-// qubits). Wider ones count as not unitary.
-constexpr int kMaxUnitaryTest = 4;
-
 // An op on physical bits (bit b = wire n-1-b), before tiling.
 struct LOp {
     uint32_t kind = TOP_DIAG;
@@ -46,9 +39,9 @@ struct LOp {
     bool is_swap() const;
     // TF_DOT_X / TF_DOT_Y / TF_DOT_Z of a dot's operator, or 0
     uint32_t dot_class() const;
-    // U^dagger U = 1 (of the operator on its targets) to tol; false also for
-    // dense operators on more than kMaxUnitaryTest bits
-    bool is_unitary(double tol) const;
+    // U U^dagger = 1 (of the operator on its targets) to tol; false also for
+    // dense operators on more than max_k bits
+    bool is_unitary(double tol, int max_k) const;
 };
 
 inline int phys_bit(int n, uint32_t wire) { return n - 1 - static_cast<int>(wire); }
@@ -163,6 +156,13 @@ struct PlanConfig {
     // for a matrix that came in single precision, complex64 states), with room
     // for a few products; past it a dot would be off by more than its rounding.
     double unitary_tol() const { return keep_grouping ? 1e-6 : 1e-12; }
+    // Dense operators on up to this many bits are tested for being unitary in
+    // programs with dots (each time the program comes); wider ones count as not
+    // unitary, which no dot passes. The test takes 2, 12 and 86 us of
+    // host time on four, five and six bits. What it may save is a pass of the
+    // dots alone: eight operators in a gradient cost 6 us each on 12 to 18
+    // qubits without the test, 70 at 22 and four times that at 24.
+    int max_unitary_test() const { return n < 20 ? 4 : n < 23 ? 5 : 6; }
     // choose each pass's tile bits by lookahead (the bits that let the most
     // work run) instead of taking the first ready op's bits
     bool lookahead = false;
